@@ -11,7 +11,7 @@
 // Layouts: hidden [T, d] bf16, weight [d, V] bf16 (the reference's
 // [d_model, vocab] matrix), targets [T] int64 (ignore_index or 0 <= t < V).
 //
-// Decomposition.  The logits are tiles of the persistent GEMM of gemm_tn.h in
+// Decomposition.  The logits are tiles of the persistent GEMM of gemm_core.h in
 // its single-matrix layout (256 tokens x 256 vocabulary entries per
 // workgroup, 64 entries per wave); the D tiles give a lane one token and 32
 // of its wave's 64 entries, so per-token reductions are in-lane plus one
@@ -27,7 +27,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
-#include "gemm_tn.h"
+#include "gemm_core.h"
 
 namespace mm1 {
 
@@ -40,67 +40,72 @@ __device__ __forceinline__ float shfl_xor32(float v) { return __shfl_xor(v, 32);
 
 }  // namespace
 
-// Partials: part[t][blk] = (max, sum of exp(l - max)) over vocabulary block blk
+// Partials: part[blk][t] = (max, sum of exp(l - max)) over vocabulary block blk
 // (64 entries, blk = 4 * column block + wave column), (-inf, 0) for a block
-// beyond the vocabulary.  tlogit[t] = the logit of column targets[t], or of
-// column 0 when the target is negative (ignore_index) or >= V, as the
-// reference's gather over targets.clamp(min=0); written by the one lane that
-// holds that column.
+// beyond the vocabulary (a whole block is inside or beyond it: V is a
+// multiple of 128); token-minor, so a wave's 32 tokens leave as one 256-byte
+// run.  tlogit[t] = the logit of column targets[t], or of column 0 when the
+// target is negative (ignore_index) or >= V, as the reference's gather over
+// targets.clamp(min=0); written by the one lane that holds that column.
+// Bound by the GEMM core; 2.05 -> 1.63 ms at 16,384 x 1280 x 49152 (1.26
+// PFLOP/s), 125 -> 106 us at 1,000 tokens, with this core, whole-block vocabulary
+// tests instead of one per logit, and token-minor partials.
 __global__ __launch_bounds__(512, 1) void lm_lse_partial_kernel(
     const __bf16* __restrict__ h, const __bf16* __restrict__ w, const long long* __restrict__ targets,
     float2* __restrict__ part, float* __restrict__ tlogit, int T, int d, int V, int n_mblk, int n_nblk) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wv & 1, wn = wv >> 1, hh = lane >> 5;
-  const gemm::Problem p{h, w, w, T, d, V, V, n_mblk, n_nblk};
-  const int n_part = 4 * n_nblk;
-  gemm::run<false>(p, smem, [](int, int) {}, [&](int mb, int nb, f32x16 (&acc)[2][4]) {
+  const gemm::Problem p{{h, d, T}, {w, V, V}, w, 0, d, n_mblk, n_nblk};
+  // the gathered column of each of the lane's tokens, loaded at the tile's
+  // first window (the loads land during the products)
+  int tcol[4];
+  auto pro = [&](int mb, int) MM1_INLINE {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const long long t = targets != nullptr ? targets[min(mb * gemm::BM + 128 * wm + 32 * i + (lane & 31), T - 1)] : 0;
+      tcol[i] = t < 0 || t >= V ? 0 : (int)t;     // the reference gathers column clamp(t, min=0)
+    }
+  };
+  gemm::run<gemm::ROW, gemm::COL, false, gemm::Wide256, gemm::WholeTiles>(p, smem, pro, [&](int mb, int nb, f32x16 (&acc)[2][4], int) MM1_INLINE {
     const int v0 = nb * 256 + 64 * wn;             // this wave's 64 vocabulary entries
+    const bool inside = v0 < V;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int tok = mb * gemm::BM + 128 * wm + 32 * i + (lane & 31);
-      float m = -INFINITY;
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int v = v0 + 32 * b + 8 * (r >> 2) + 4 * hh + (r & 3);
-          if (v < V) m = fmaxf(m, acc[b][i][r]);
-        }
-      }
-      m = fmaxf(m, shfl_xor32(m));
-      float s = 0.f;
-      if (m > -INFINITY) {
-        const float ms = m * kLog2e;
+      float m = -INFINITY, s = 0.f;
+      if (inside) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int v = v0 + 32 * b + 8 * (r >> 2) + 4 * hh + (r & 3);
-            if (v < V) s += exp2_fast(acc[b][i][r] * kLog2e - ms);
+          for (int r = 0; r < 16; ++r) m = fmaxf(m, acc[b][i][r]);
+        }
+        m = fmaxf(m, shfl_xor32(m));
+        if (m > -INFINITY) {
+          const float ms = m * kLog2e;
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s += exp2_fast(fmaf(acc[b][i][r], kLog2e, -ms));
           }
         }
+        s += shfl_xor32(s);
       }
-      s += shfl_xor32(s);
       if (tok < T) {
-        if (hh == 0) part[(long)tok * n_part + 4 * nb + wn] = make_float2(m, s);
-        if (targets != nullptr) {
-          long long tv = targets[tok];
-          if (tv < 0 || tv >= V) tv = 0;     // the reference gathers column clamp(t, min=0)
-          if (tv >= v0 && tv < v0 + 64) {
-            const int rel = (int)(tv - v0);
-            const int b = rel >> 5, rr = rel & 31;       // block, row inside the D tile
-            if (((rr >> 2) & 1) == hh) {
-              const int reg = 4 * (rr >> 3) + (rr & 3);
-              float val = 0.f;
+        if (hh == 0) part[(long)(4 * nb + wn) * T + tok] = make_float2(m, s);
+        const int rel = tcol[i] - v0;
+        if (targets != nullptr && inside && rel >= 0 && rel < 64) {
+          const int b = rel >> 5, rr = rel & 31;       // block, row inside the D tile
+          if (((rr >> 2) & 1) == hh) {
+            const int reg = 4 * (rr >> 3) + (rr & 3);
+            float val = 0.f;
 #pragma unroll
-              for (int bb = 0; bb < 2; ++bb) {
+            for (int bb = 0; bb < 2; ++bb) {
 #pragma unroll
-                for (int q = 0; q < 16; ++q)
-                  if (bb == b && q == reg) val = acc[bb][i][q];
-              }
-              tlogit[tok] = val;
+              for (int q = 0; q < 16; ++q)
+                if (bb == b && q == reg) val = acc[bb][i][q];
             }
+            tlogit[tok] = val;
           }
         }
       }
@@ -108,11 +113,12 @@ __global__ __launch_bounds__(512, 1) void lm_lse_partial_kernel(
   });
 }
 
-// One wave per token: lse = m* + ln(sum_j s_j exp(m_j - m*)) over the token's
-// partials, in one pass: each lane folds partials lane, lane + 64, ... into a
-// running (max, sum) in index order, then the lanes' pairs merge by a fixed
-// shuffle tree (deterministic); the token loss is lse - target_logit (0 for
-// ignored or out-of-range targets).
+// lse = m* + ln(sum_j s_j exp(m_j - m*)) over a token's partials, in one pass
+// and a fixed order (deterministic): a workgroup owns 16 tokens and splits
+// their partials 64 ways (thread t: token t % 16, partials t / 16, t / 16 +
+// 64, ...); the pairs then merge by a fixed tree, in the wave by shuffles and
+// across the 16 waves through LDS.  The token loss is lse - target_logit (0
+// for ignored or out-of-range targets).
 __device__ __forceinline__ void lse_merge(float& m, float& s, float m2, float s2) {
   const float mn = fmaxf(m, m2);
   if (mn == -INFINITY) return;                    // both empty
@@ -120,38 +126,43 @@ __device__ __forceinline__ void lse_merge(float& m, float& s, float m2, float s2
   m = mn;
 }
 
-__global__ __launch_bounds__(256) void lm_lse_combine_kernel(
+constexpr int COMBINE_THREADS = 1024, COMBINE_TOKENS = 16, COMBINE_SPLIT = COMBINE_THREADS / COMBINE_TOKENS;
+
+__global__ __launch_bounds__(COMBINE_THREADS) void lm_lse_combine_kernel(
     const float2* __restrict__ part, const float* __restrict__ tlogit, const long long* __restrict__ targets,
     float* __restrict__ lse, float* __restrict__ loss, int T, int V, int n_part, long long ignore_index) {
-  const int lane = threadIdx.x & 63;
-  const int tok = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (tok >= T) return;
-  const float2* row = part + (long)tok * n_part;
+  __shared__ float2 merged[COMBINE_THREADS / 64][COMBINE_TOKENS];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int tok = blockIdx.x * COMBINE_TOKENS + (lane & 15);
+  const float2* col = part + min(tok, T - 1);
   float m = -INFINITY, s = 0.f;
-  int j = lane;
-  for (; j + 192 < n_part; j += 256) {            // four loads in flight per lane
+  int j = threadIdx.x >> 4;
+  for (; j + 3 * COMBINE_SPLIT < n_part; j += 4 * COMBINE_SPLIT) {   // four loads in flight per lane
     float2 v[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = row[j + 64 * u];
+    for (int u = 0; u < 4; ++u) v[u] = col[(long)(j + u * COMBINE_SPLIT) * T];
 #pragma unroll
     for (int u = 0; u < 4; ++u) lse_merge(m, s, v[u].x, v[u].y);
   }
-  for (; j < n_part; j += 64) {
-    const float2 v = row[j];
+  for (; j < n_part; j += COMBINE_SPLIT) {
+    const float2 v = col[(long)j * T];
     lse_merge(m, s, v.x, v.y);
   }
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
+  for (int o = 16; o <= 32; o <<= 1) {
     const float m2 = __shfl_xor(m, o), s2 = __shfl_xor(s, o);
     lse_merge(m, s, m2, s2);
   }
-  if (lane == 0) {
-    const float l = m + log2f(s) * kLn2;
-    lse[tok] = l;
-    if (loss != nullptr) {
-      const long long tv = targets[tok];
-      loss[tok] = (tv != ignore_index && tv >= 0 && tv < V) ? l - tlogit[tok] : 0.f;
-    }
+  if (lane < COMBINE_TOKENS) merged[w][lane] = make_float2(m, s);
+  __syncthreads();
+  if (threadIdx.x >= COMBINE_TOKENS || tok >= T) return;
+#pragma unroll
+  for (int u = 1; u < COMBINE_THREADS / 64; ++u) lse_merge(m, s, merged[u][lane].x, merged[u][lane].y);
+  const float l = m + log2f(s) * kLn2;
+  lse[tok] = l;
+  if (loss != nullptr) {
+    const long long tv = targets[tok];
+    loss[tok] = (tv != ignore_index && tv >= 0 && tv < V) ? l - tlogit[tok] : 0.f;
   }
 }
 
@@ -159,48 +170,60 @@ __global__ __launch_bounds__(256) void lm_lse_combine_kernel(
 // columns of weight + v0; out[t][v] (row stride ld) = bf16((exp(l - lse[t]) -
 // [v0 + v == target[t]]) * scale) for valid targets, 0 for ignored ones.
 // `scale` is a device scalar (the loss gradient over the valid count).
+template <bool NT>
 __global__ __launch_bounds__(512, 1) void lm_dlogits_kernel(
     const __bf16* __restrict__ h, const __bf16* __restrict__ w, const long long* __restrict__ targets,
     const float* __restrict__ lse, const float* __restrict__ scale, __bf16* __restrict__ out, long ld,
     int T, int d, int V, int v0, int vn, long long ignore_index, int n_mblk, int n_nblk) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wv & 1, wn = wv >> 1;
-  const gemm::Problem p{h, w + v0, w + v0, T, d, V, vn, n_mblk, n_nblk};
+  const gemm::Problem p{{h, d, T}, {w + v0, V, vn}, w, 0, d, n_mblk, n_nblk};
   const float sc = *scale;
   // the rows go out through 4 KiB per wave above the GEMM's ring
-  char* stage = smem + gemm::LDS_BYTES + gemm::STAGE_BYTES * wv;
-  // Targets and lse of the tile's tokens, loaded at its first k step (the
+  char* stage = smem + gemm::Wide256::RING + gemm::Wide256::STAGE_BYTES * wv;
+  // Target column (of this chunk; out of its range when there is none),
+  // factor and lse of the tile's tokens, loaded at its first window (the
   // loads land during the products, not in the epilogue).
-  long long tv[4];
-  float l2[4];
-  auto pro = [&](int mb, int) {
+  int tcol[4];
+  float coef[4], l2[4];
+  auto pro = [&](int mb, int) MM1_INLINE {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int tok = min(mb * gemm::BM + 128 * wm + 32 * i + (lane & 31), T - 1);
-      tv[i] = targets[tok];
+      const long long t = targets[tok];
+      const bool valid = t != ignore_index && t >= 0 && t < V;
+      tcol[i] = valid ? (int)t - v0 : -1;
+      coef[i] = valid ? sc : 0.f;
       l2[i] = lse[tok] * kLog2e;
     }
   };
-  gemm::run<false>(p, smem, pro, [&](int mb, int nb, f32x16 (&acc)[2][4]) {
+  gemm::run<gemm::ROW, gemm::COL, false, gemm::Wide256, gemm::WholeTiles>(p, smem, pro, [&](int mb, int nb, f32x16 (&acc)[2][4], int) MM1_INLINE {
     const int c0 = nb * 256 + 64 * wn;             // this wave's first column of the chunk
     const long tok0 = (long)mb * gemm::BM + 128 * wm;
-    auto val = [&](int i, int b, int q) {
-      const long long t = tv[i];
-      const bool valid = t != ignore_index && t >= 0 && t < V;
-      const float coef = valid ? sc : 0.f;
-      const long long tcol = t - v0;               // the target's column in this chunk
-      const int c = c0 + 32 * b + 8 * q + 4 * (lane >> 5);
-      bf16x4 o;
+    // the target's column among the wave's 64, counted from the lane's first;
+    // few waves hold the target of any of their tokens
+    int rel[4];
+    bool any[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float pr = exp2_fast(acc[b][i][4 * q + e] * kLog2e - l2[i]);
-        if (c + e == tcol) pr -= 1.f;
-        o[e] = (__bf16)(pr * coef);
+    for (int i = 0; i < 4; ++i) {
+      rel[i] = tcol[i] - c0 - 4 * (lane >> 5);
+      any[i] = __any(rel[i] >= 0 && rel[i] < 64);
+    }
+    auto val = [&](int i, int b, int q) {
+      bf16x4 o;
+      float pr[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pr[e] = exp2_fast(fmaf(acc[b][i][4 * q + e], kLog2e, -l2[i]));
+      if (any[i]) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pr[e] -= rel[i] == 32 * b + 8 * q + e ? 1.f : 0.f;
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (__bf16)(pr[e] * coef[i]);
       return o;
     };
-    gemm::store_rows128(
+    gemm::store_rows128<NT>(
         stage, lane, val,
         [&](int r) -> __bf16* { return tok0 + r < T ? out + (tok0 + r) * ld + c0 : nullptr; },
         [&](int c) { return c0 + 8 * c < vn; });
@@ -230,17 +253,17 @@ hipError_t launch_lm_lse(const void* hidden, const void* weight, const long long
   hipError_t e = gemm_geometry(T, V, n_mblk, n_nblk, grid);
   if (e != hipSuccess) return e;
   e = hipFuncSetAttribute(reinterpret_cast<const void*>(lm_lse_partial_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm::LDS_BYTES);
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm::Wide256::RING);
   if (e != hipSuccess) return e;
   const int n_part = 4 * n_nblk;
   auto part = static_cast<float2*>(workspace);
   float* tl = tlogit_out != nullptr
                   ? tlogit_out
                   : reinterpret_cast<float*>(static_cast<char*>(workspace) + (size_t)T * n_part * sizeof(float2));
-  hipLaunchKernelGGL(lm_lse_partial_kernel, dim3(grid), dim3(512), gemm::LDS_BYTES, stream,
+  hipLaunchKernelGGL(lm_lse_partial_kernel, dim3(grid), dim3(512), gemm::Wide256::RING, stream,
                      static_cast<const __bf16*>(hidden), static_cast<const __bf16*>(weight), targets, part, tl,
                      T, d, V, n_mblk, n_nblk);
-  hipLaunchKernelGGL(lm_lse_combine_kernel, dim3((T + 3) / 4), dim3(256), 0, stream, part, tl, targets, lse,
+  hipLaunchKernelGGL(lm_lse_combine_kernel, dim3((T + COMBINE_TOKENS - 1) / COMBINE_TOKENS), dim3(COMBINE_THREADS), 0, stream, part, tl, targets, lse,
                      targets != nullptr ? loss : nullptr, T, V, n_part, ignore_index);
   return hipGetLastError();
 }
@@ -251,11 +274,15 @@ hipError_t launch_lm_dlogits(const void* hidden, const void* weight, const long 
   int n_mblk, n_nblk, grid;
   hipError_t e = gemm_geometry(T, vn, n_mblk, n_nblk, grid);
   if (e != hipSuccess) return e;
-  const size_t lds = gemm::LDS_BYTES + 8 * gemm::STAGE_BYTES;   // ring + the epilogue's staging
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(lm_dlogits_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const size_t lds = gemm::Wide256::LDS_BYTES;   // ring + the epilogue's staging
+  // d_logits too large for the memory-side cache leave with non-temporal
+  // stores (16,384 tokens, whole vocabulary: 2.03 -> 1.75 ms with the
+  // core of gemm_core.h); at 1,000 tokens (98 MB) the product that reads them next is 28 us
+  // faster when they were stored through the caches.
+  auto kern = (long)T * vn * 2 > gemm::CACHED_BYTES ? lm_dlogits_kernel<true> : lm_dlogits_kernel<false>;
+  e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(lm_dlogits_kernel, dim3(grid), dim3(512), lds, stream,
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, stream,
                      static_cast<const __bf16*>(hidden), static_cast<const __bf16*>(weight), targets, lse, scale,
                      static_cast<__bf16*>(dlogits), ld, T, d, V, v0, vn, ignore_index, n_mblk, n_nblk);
   return hipGetLastError();
