@@ -35,6 +35,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib
+from . import gemm
 from . import tuned
 from .harness import Report, compare, needs_gpu, time_cuda
 from .harness import main as harness_main
@@ -560,28 +561,30 @@ def apply_rope(x, cos, sin):
 _HIP_BACKENDS = ("hip", "tilelang")
 
 
-# Token chunks of the projections' weight-gradient GEMMs (wgrad.py): 8
-# measured fastest for wq|wk|wv and wo at 16,384 tokens.
+# Token chunks of the projections' weight-gradient GEMMs where hipBLASLt runs
+# them (wgrad.py): 8 measured fastest of the chunk counts.
 PROJ_DW_CHUNKS = 8
 
 
 class BF16Linear(torch.autograd.Function):
-    """y = x W^T of the sublayer's projections under bf16 autocast, with the
-    weight gradient in the GEMM form hipBLASLt runs fastest on gfx950:
-      dX = dY W, as autograd computes it;
-      dW = sum over PROJ_DW_CHUNKS token chunks of dY_c^T X_c, each a GEMM with
-           fp32 outputs, summed in fp32 (the reference's autocast graph rounds
-           the one bf16 GEMM's dW to bf16 before its fp32 cast, AT:470-472,
-           :518; this dW is the same sum without that rounding).
+    """y = x W^T of the sublayer's projections under bf16 autocast, each product
+    on the GEMM core where that is the faster choice (gemm.py):
+      y = x W^T and dX = dY W, as autograd computes them;
+      dW = dY^T X with fp32 sums and fp32 output (wgrad.py; the reference's
+           autocast graph rounds the bf16 GEMM's dW to bf16 before its fp32
+           cast, AT:470-472, :518; this dW is the same sum without that
+           rounding).
     x may be fp32 or bf16 (cast here, as autocast would); w is the fp32
-    parameter (cast here; its gradient is returned in fp32).  The forward is
-    the same F.linear on the same bf16 operands as the module's."""
+    parameter (cast here; its gradient is returned in fp32)."""
 
     @staticmethod
     def forward(ctx, x, w):
         xb, wb = x.to(DTYPE), w.to(DTYPE)
         ctx.save_for_backward(xb, wb)
         ctx.x_dtype, ctx.w_dtype = x.dtype, w.dtype
+        x2 = xb.reshape(-1, xb.shape[-1])
+        if gemm.applies(x2, wb):
+            return gemm.product(x2, wb).reshape(*xb.shape[:-1], wb.shape[0])
         return F.linear(xb, wb)
 
     @staticmethod
@@ -592,7 +595,8 @@ class BF16Linear(torch.autograd.Function):
         x2 = xb.reshape(-1, k)
         dx = dw = None
         if ctx.needs_input_grad[0]:
-            dx = (dy2 @ wb).reshape(*dy.shape[:-1], k).to(ctx.x_dtype)
+            dx = gemm.product(dy2, wb.t()) if gemm.applies(dy2, wb.t()) else dy2 @ wb
+            dx = dx.reshape(*dy.shape[:-1], k).to(ctx.x_dtype)
         if ctx.needs_input_grad[1]:
             dw = wgrad(dy2, x2, PROJ_DW_CHUNKS).to(ctx.w_dtype)
         return dx, dw

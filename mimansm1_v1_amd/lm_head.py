@@ -16,8 +16,8 @@ The kernels are the gfx950 HIP kernels of ``csrc/lm_head.hip`` behind the C ABI
 (``include/mm1_lm_head.h``): the forward computes, in one GEMM pass over the
 vocabulary, each token's log-sum-exp and target logit without storing the
 [tokens, vocab] logits; the backward computes bf16 d_logits one vocabulary
-chunk at a time in a second GEMM pass and hands them to two hipBLASLt GEMMs
-(d_hidden, d_weight).  On a 288 GB MI355X the default chunk is the whole
+chunk at a time in a second GEMM pass and multiplies them into d_hidden and
+d_weight (gemm.py, or hipBLASLt at the sizes it is faster at).  On a 288 GB MI355X the default chunk is the whole
 vocabulary (1.6 GB of bf16 d_logits at 8 x 2048 tokens), where the
 reference's 4096-entry chunks were sized for a much smaller card.  Without the
 built library the kernel entry points raise; there is no CPU fallback.
@@ -32,6 +32,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib
+from . import gemm
 from . import tuned
 from .harness import Report, compare, needs_gpu, time_cuda
 from .harness import main as harness_main
@@ -156,6 +157,11 @@ def gather_target_logits(hidden, weight, targets):
     return (hidden.to(acc) * rows.to(acc)).sum(-1)
 
 
+def _matmul(x, w):
+    """x w^T on the GEMM core where it applies (gemm.py), else torch's GEMM."""
+    return gemm.product(x, w) if gemm.applies(x, w) else x @ w.t()
+
+
 class FusedCrossEntropy(torch.autograd.Function):
     """Same signature and returns as LM:193-243: the mean cross entropy over
     tokens whose target is not IGNORE_INDEX (0 when there are none).  bf16
@@ -188,14 +194,14 @@ class FusedCrossEntropy(torch.autograd.Function):
         if chunk >= vocab:
             # the whole vocabulary at once: two plain GEMMs on the bf16 d_logits
             dl = kernel.dlogits(hidden, weight, targets, lse, scale, 0, vocab)
-            return dl @ weight.t(), hidden.t() @ dl, None, None
+            return _matmul(dl, weight), _matmul(hidden.t(), dl.t()), None, None
         d_weight = torch.empty_like(weight)
         d_hidden = torch.zeros(tokens, d_model, dtype=torch.float32, device=hidden.device)
         for start in range(0, vocab, chunk):
             stop = min(start + chunk, vocab)
             dl = kernel.dlogits(hidden, weight, targets, lse, scale, start, stop - start)
-            d_hidden += (dl @ weight[:, start:stop].t()).float()
-            d_weight[:, start:stop] = hidden.t() @ dl
+            d_hidden += _matmul(dl, weight[:, start:stop]).float()
+            d_weight[:, start:stop] = _matmul(hidden.t(), dl.t())
         return d_hidden.to(hidden.dtype), d_weight, None, None
 
 

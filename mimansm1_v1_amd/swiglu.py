@@ -14,8 +14,9 @@ Drop-in surface (same names, arguments, layouts and return values):
 The kernels are the gfx950 HIP kernels of ``csrc/swiglu.hip`` behind the C ABI
 (``include/mm1_swiglu.h``): the gate/up GEMM with the SwiGLU epilogue fused
 (one launch writes gate, up and act for training), and the elementwise
-gradient.  The down projection and the backward's GEMMs are hipBLASLt through
-torch, as in the reference.  Without the built library every kernel entry
+gradient.  The down projection and the backward's GEMMs run on the same GEMM
+core (gemm.py) where it is the faster choice, else on hipBLASLt through torch,
+as in the reference.  Without the built library every kernel entry
 point raises; nothing falls back to another implementation.
 """
 from __future__ import annotations
@@ -29,6 +30,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib
+from . import gemm
 from . import tuned
 from .harness import Report, compare, needs_gpu, time_cuda
 from .harness import main as harness_main
@@ -198,21 +200,27 @@ def warmup(tokens, cfg=None):
     get_kernel("grad", tokens, cfg.ffn_hidden)
 
 
+def _matmul(x, w):
+    """x w^T on the GEMM core where it applies (gemm.py), else torch's GEMM."""
+    return gemm.product(x, w) if gemm.applies(x, w) else x @ w.t()
+
+
 class FusedSwiGLU(torch.autograd.Function):
     """Same signature and returns as SW:276-301.  Forward: one HIP launch for
     gate, up and act (the reference's split kernel plus its two elementwise
     torch ops), then act @ w_down.  Backward: d_act = grad_out @ w_down^T, the
     HIP gradient kernel writing [d_gate | d_up] into one [T, 2F] buffer, and
     the reference's GEMMs with the two gate/up weight gradients from one
-    product (x^T [d_gate | d_up]), d_x accumulated in one addmm, and the
-    down-projection weight gradient over two token chunks (wgrad.py)."""
+    product (x^T [d_gate | d_up]), d_x from one product over the joined
+    [w_gate | w_up], and the weight gradients summed in fp32 (wgrad.py).  The
+    products run on the GEMM core (gemm.py) at the sizes it is faster at."""
 
     @staticmethod
     def forward(ctx, x, w_gate, w_up, w_down):
         tokens, d_model = x.shape
         ffn = w_gate.shape[1]
         gate, up, act = get_kernel("train", tokens, d_model, ffn)(x, w_gate, w_up)
-        out = act @ w_down
+        out = _matmul(act, w_down.t())
         ctx.save_for_backward(x, w_gate, w_up, w_down, gate, up, act)
         return out
 
@@ -223,15 +231,23 @@ class FusedSwiGLU(torch.autograd.Function):
         grad_out = grad_out.contiguous()
         if grad_out.dtype != x.dtype:
             grad_out = grad_out.to(x.dtype)
-        d_act = grad_out @ w_down.t()
+        d_act = _matmul(grad_out, w_down)
         d_gu = torch.empty(tokens, 2 * ffn, dtype=x.dtype, device=x.device)
         d_gate, d_up = get_kernel("grad", tokens, ffn)(d_act, gate, up, out=d_gu)
-        d_x = torch.addmm(d_gate @ w_gate.t(), d_up, w_up.t())
-        d_w = x.t() @ d_gu
-        # fp32 sum of two token chunks (wgrad.py), rounded to the weight's
-        # dtype once, as the single bf16 GEMM rounds it
-        d_w_down = wgrad(act, grad_out, DOWN_DW_CHUNKS).to(w_down.dtype)
-        return d_x, d_w[:, :ffn], d_w[:, ffn:], d_w_down
+        # d_x = [d_gate | d_up] [w_gate | w_up]^T as one product over 2F
+        if gemm.applies_joined(d_gu, w_gate, w_up):
+            d_x = gemm.product(d_gu, w_gate, w1=w_up)
+        else:
+            d_x = torch.addmm(d_gate @ w_gate.t(), d_up, w_up.t())
+        if gemm.applies(x.t(), d_gu.t()):
+            d_w_gate, d_w_up = gemm.product(x.t(), d_gu.t(), split=ffn)
+        else:
+            d_w = x.t() @ d_gu
+            d_w_gate, d_w_up = d_w[:, :ffn], d_w[:, ffn:]
+        # fp32 sums (wgrad.py), rounded to the weight's dtype once, as the
+        # single bf16 GEMM rounds it
+        d_w_down = wgrad(act, grad_out, DOWN_DW_CHUNKS, w_down.dtype)
+        return d_x, d_w_gate, d_w_up, d_w_down
 
 
 def fused_swiglu(x, w_gate, w_up, w_down):

@@ -1,0 +1,91 @@
+"""The plain bf16 products (mimansm1_v1_amd/gemm.py) against fp64 products of
+the same operands: every layout, ragged edges of the tiles, both tile widths,
+the split along K, joined weights, halved outputs and fp32 outputs."""
+import pytest
+import torch
+
+from mimansm1_v1_amd import _lib, gemm
+
+pytestmark = pytest.mark.gpu
+
+
+def operand(rows, k, col, gen, dev, pad=0):
+    """[rows, K], stored with K contiguous or (col) outermost, row stride padded."""
+    inner, outer = (rows, k) if col else (k, rows)
+    t = torch.randn(outer, inner + pad, device=dev, generator=gen).to(torch.bfloat16)[:, :inner]
+    return t.t() if col else t
+
+
+def check(out, x, w):
+    """Within the rounding of the output plus that of fp32 sums over K: |err| <=
+    u |exact| + K 2^-24 sum_k |x w|, u = 2^-8 (bf16, one ulp) or 0."""
+    xd, wd = x.double().contiguous(), w.double().contiguous()
+    exact = xd @ wd.t().contiguous()
+    size = xd.abs() @ wd.abs().t().contiguous()
+    u = 2.0 ** -8 if out.dtype == torch.bfloat16 else 0.0
+    over = ((out.double() - exact).abs() - u * exact.abs() - x.shape[1] * 2.0 ** -24 * size).max().item()
+    assert over <= 0, over
+
+
+# (M, N, K): smallest; ragged rows and columns of a tile; several tiles; a
+# 320-column width; few tiles over a long K (split over all CUs, runs of one
+# and of two tiles); fewer window pairs than CUs (empty runs); 257 tiles (one left over)
+SHAPES = [(8, 8, 128), (256, 256, 128), (264, 520, 256), (776, 1288, 384), (1000, 320, 640),
+          (512, 1280, 8192), (264, 264, 16384), (8, 8, 16384), (1280, 640, 6144), (65792, 256, 256)]
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_products_vs_fp64(hip_device, M, N, K, layout):
+    gen = torch.Generator(device=hip_device).manual_seed(M + N + K)
+    x = operand(M, K, layout == "tn", gen, hip_device)
+    w = operand(N, K, layout != "nt", gen, hip_device)
+    for dtype in (torch.bfloat16, torch.float32):
+        out = gemm.product(x, w, out_dtype=dtype)
+        check(out, x, w)
+        assert torch.equal(out, gemm.product(x, w, out_dtype=dtype))
+
+
+@pytest.mark.parametrize("M", [1, 77, 255, 257, 333])
+def test_ragged_rows_and_padded_strides(hip_device, M):
+    gen = torch.Generator(device=hip_device).manual_seed(M)
+    for col in (False, True):
+        x = operand(M, 256, False, gen, hip_device, pad=8)
+        w = operand(328, 256, col, gen, hip_device, pad=16)
+        check(gemm.product(x, w), x, w)
+
+
+@pytest.mark.parametrize("T,d,F", [(300, 640, 128), (4096, 1280, 3328), (2048, 256, 4160)])
+def test_joined_weights_and_split_output(hip_device, T, d, F):
+    gen = torch.Generator(device=hip_device).manual_seed(T)
+    d_gu = operand(T, 2 * F, False, gen, hip_device)
+    wg, wu = (operand(d, F, False, gen, hip_device) for _ in range(2))
+    check(gemm.product(d_gu, wg, w1=wu), d_gu, torch.cat((wg, wu), dim=1))
+    if T % 128:
+        return
+    x = operand(d, T, True, gen, hip_device)
+    lo, hi = gemm.product(x, d_gu.t(), split=F)
+    check(lo, x, d_gu.t()[:F])
+    check(hi, x, d_gu.t()[F:])
+
+
+def test_c_abi_refuses_what_the_kernels_do_not_take(hip_device):
+    lib = _lib.load()
+    t = torch.zeros(512 * 512, dtype=torch.bfloat16, device=hip_device)
+    p = t.data_ptr()
+
+    def call(x=p, lx=0, ldx=256, w=p, lw=0, ldw=256, w1=None, cut=0, out=p, out1=None, n_cut=0, ldo=256,
+             M=64, N=64, K=256):
+        return lib.mm1_gemm(x, lx, ldx, w, lw, ldw, w1, cut, out, out1, n_cut, ldo, 0, None, 0, M, N, K, None)
+
+    assert call(x=None) == -1
+    for bad in (dict(K=192), dict(N=60), dict(lx=1), dict(lx=2), dict(ldx=128), dict(ldw=252), dict(ldo=32),
+                dict(cut=64), dict(w1=p, cut=32), dict(out1=p, n_cut=32), dict(M=0), dict(lx=1, lw=1, M=60),
+                dict(M=1 << 29), dict(ldx=1 << 22)):
+        assert call(**bad) == -2, bad
+    assert call(x=p + 2) == -6
+    need = lib.mm1_gemm_workspace_size(512, 1280, 8192)
+    assert need > 0
+    big = torch.zeros(1280 * 8192, dtype=torch.bfloat16, device=hip_device).data_ptr()
+    assert lib.mm1_gemm(big, 0, 8192, big, 0, 8192, None, 0, big, None, 0, 1280, 0, None, 0, 512, 1280, 8192,
+                        None) == -4
