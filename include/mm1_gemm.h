@@ -36,7 +36,8 @@ size_t mm1_gemm_workspace_size(int M, int N, int K);
  *   out1, n_cut: with out1 != NULL, out holds the columns below n_cut and out1
  *     (same stride) the others; n_cut a multiple of 64.  Else n_cut = 0.
  * x ROW with w ROW or COL, or both COL (MM1_E_SHAPE for x COL with w ROW).
- * M, N, K >= 1, K a multiple of 128, N a multiple of 8 (and M when x is COL),
+ * M, N, K >= 1, K a multiple of 128 unless both are COL (then any K, at most
+ * 2^28), N a multiple of 8 (and M when x is COL),
  * every stride a multiple of 8 and at least its row's length, 16-byte aligned
  * pointers; the bytes of 256 rows of a ROW operand and of 64 rows of a COL
  * operand below 2^31, M and N at most 2^28, at most 2^24 output tiles of

@@ -55,6 +55,15 @@ int mm1_lm_head_dlogits(const void* hidden, const void* weight, const long long*
                         const float* lse, const float* scale, void* d_logits, long ld,
                         int T, int d_model, int vocab, int v0, int vn, void* stream);
 
+/* The same two calls for a weight stored [vocab, d_model] (an embedding
+ * matrix as it lies in memory: a head tied to it needs no transposed copy). */
+int mm1_lm_head_lse_rows(const void* hidden, const void* weight, const long long* targets, long long ignore_index,
+                         float* lse, float* target_logit, float* loss, void* workspace, size_t workspace_bytes,
+                         int T, int d_model, int vocab, void* stream);
+int mm1_lm_head_dlogits_rows(const void* hidden, const void* weight, const long long* targets,
+                             long long ignore_index, const float* lse, const float* scale, void* d_logits, long ld,
+                             int T, int d_model, int vocab, int v0, int vn, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -57,6 +57,10 @@ SIGNATURES = {
                                  _c_int, _c_int, _c_int, _vp]),
     "mm1_lm_head_dlogits": (_c_int, [_vp, _vp, _vp, ctypes.c_longlong, _vp, _vp, _vp, ctypes.c_long,
                                      _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
+    "mm1_lm_head_lse_rows": (_c_int, [_vp, _vp, _vp, ctypes.c_longlong, _vp, _vp, _vp, _vp, _c_size,
+                                      _c_int, _c_int, _c_int, _vp]),
+    "mm1_lm_head_dlogits_rows": (_c_int, [_vp, _vp, _vp, ctypes.c_longlong, _vp, _vp, _vp, ctypes.c_long,
+                                          _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
     "mm1_gemm_workspace_size": (_c_size, [_c_int, _c_int, _c_int]),
     "mm1_gemm": (_c_int, [_vp, _c_int, ctypes.c_long, _vp, _c_int, ctypes.c_long, _vp, _c_int, _vp, _vp, _c_int,
                           ctypes.c_long, _c_int, _vp, _c_size, _c_int, _c_int, _c_int, _vp]),

@@ -43,10 +43,11 @@ hipError_t launch_swiglu_gate_up(const void* x, const void* wg, const void* wu, 
 hipError_t launch_swiglu_grad(const void* dact, const void* gate, const void* up, void* dgate, void* dup,
                               int T, int F, long ld_out, hipStream_t stream);
 size_t lm_head_workspace_bytes(int T, int V);
-hipError_t launch_lm_lse(const void* hidden, const void* weight, const long long* targets, long long ignore_index,
+hipError_t launch_lm_lse(const void* hidden, const void* weight, bool vocab_rows, const long long* targets,
+                         long long ignore_index,
                          float* lse, float* tlogit_out, float* loss, void* workspace, int T, int d, int V,
                          hipStream_t stream);
-hipError_t launch_lm_dlogits(const void* hidden, const void* weight, const long long* targets,
+hipError_t launch_lm_dlogits(const void* hidden, const void* weight, bool vocab_rows, const long long* targets,
                              long long ignore_index, const float* lse, const float* scale, void* dlogits, long ld,
                              int T, int d, int V, int v0, int vn, hipStream_t stream);
 hipError_t launch_qknorm_bwd(const void* qkv, const float* wq, const float* wk, const float* cos_t,
@@ -609,34 +610,62 @@ size_t mm1_lm_head_workspace_size(int T, int vocab) {
   return mm1::lm_head_workspace_bytes(T, vocab);
 }
 
-int mm1_lm_head_lse(const void* hidden, const void* weight, const long long* targets, long long ignore_index,
-                    float* lse, float* target_logit, float* loss, void* workspace, size_t workspace_bytes,
-                    int T, int d_model, int vocab, void* stream) {
+static int lm_head_lse(const void* hidden, const void* weight, bool vocab_rows, const long long* targets,
+                       long long ignore_index, float* lse, float* target_logit, float* loss, void* workspace,
+                       size_t workspace_bytes, int T, int d_model, int vocab, void* stream) {
   if (!hidden || !weight || !lse) return MM1_E_NULL;
   if (!targets && (target_logit || loss)) return MM1_E_NULL;
   int rc = check_lm_shape(T, d_model, vocab);
   if (rc) return rc;
   if (!workspace || workspace_bytes < mm1::lm_head_workspace_bytes(T, vocab)) return MM1_E_WORKSPACE;
   if (!aligned16(hidden) || !aligned16(weight) || !aligned16(workspace)) return MM1_E_ALIGN;
-  return from_hip(mm1::launch_lm_lse(hidden, weight, targets, ignore_index, lse, target_logit, loss, workspace,
-                                     T, d_model, vocab, static_cast<hipStream_t>(stream)));
+  return from_hip(mm1::launch_lm_lse(hidden, weight, vocab_rows, targets, ignore_index, lse, target_logit, loss,
+                                     workspace, T, d_model, vocab, static_cast<hipStream_t>(stream)));
 }
 
-int mm1_lm_head_dlogits(const void* hidden, const void* weight, const long long* targets, long long ignore_index,
-                        const float* lse, const float* scale, void* d_logits, long ld,
-                        int T, int d_model, int vocab, int v0, int vn, void* stream) {
+int mm1_lm_head_lse(const void* hidden, const void* weight, const long long* targets, long long ignore_index,
+                    float* lse, float* target_logit, float* loss, void* workspace, size_t workspace_bytes,
+                    int T, int d_model, int vocab, void* stream) {
+  return lm_head_lse(hidden, weight, false, targets, ignore_index, lse, target_logit, loss, workspace,
+                     workspace_bytes, T, d_model, vocab, stream);
+}
+
+int mm1_lm_head_lse_rows(const void* hidden, const void* weight, const long long* targets, long long ignore_index,
+                         float* lse, float* target_logit, float* loss, void* workspace, size_t workspace_bytes,
+                         int T, int d_model, int vocab, void* stream) {
+  return lm_head_lse(hidden, weight, true, targets, ignore_index, lse, target_logit, loss, workspace,
+                     workspace_bytes, T, d_model, vocab, stream);
+}
+
+static int lm_head_dlogits(const void* hidden, const void* weight, bool vocab_rows, const long long* targets,
+                           long long ignore_index, const float* lse, const float* scale, void* d_logits, long ld,
+                           int T, int d_model, int vocab, int v0, int vn, void* stream) {
   if (!hidden || !weight || !targets || !lse || !scale || !d_logits) return MM1_E_NULL;
   int rc = check_lm_shape(T, d_model, vocab);
   if (rc) return rc;
   if (v0 < 0 || vn < 128 || v0 % 128 != 0 || vn % 128 != 0 || (long)v0 + vn > vocab || ld < vn || ld % 8 != 0)
     return MM1_E_SHAPE;
   if (!aligned16(hidden) || !aligned16(weight) || !aligned16(d_logits)) return MM1_E_ALIGN;
-  return from_hip(mm1::launch_lm_dlogits(hidden, weight, targets, ignore_index, lse, scale, d_logits, ld, T,
-                                         d_model, vocab, v0, vn, static_cast<hipStream_t>(stream)));
+  return from_hip(mm1::launch_lm_dlogits(hidden, weight, vocab_rows, targets, ignore_index, lse, scale, d_logits, ld,
+                                         T, d_model, vocab, v0, vn, static_cast<hipStream_t>(stream)));
+}
+
+int mm1_lm_head_dlogits(const void* hidden, const void* weight, const long long* targets, long long ignore_index,
+                        const float* lse, const float* scale, void* d_logits, long ld,
+                        int T, int d_model, int vocab, int v0, int vn, void* stream) {
+  return lm_head_dlogits(hidden, weight, false, targets, ignore_index, lse, scale, d_logits, ld, T, d_model, vocab,
+                         v0, vn, stream);
+}
+
+int mm1_lm_head_dlogits_rows(const void* hidden, const void* weight, const long long* targets,
+                             long long ignore_index, const float* lse, const float* scale, void* d_logits, long ld,
+                             int T, int d_model, int vocab, int v0, int vn, void* stream) {
+  return lm_head_dlogits(hidden, weight, true, targets, ignore_index, lse, scale, d_logits, ld, T, d_model, vocab,
+                         v0, vn, stream);
 }
 
 size_t mm1_gemm_workspace_size(int M, int N, int K) {
-  if (M < 1 || N < 1 || K < 128 || K % 128 != 0) return 0;
+  if (M < 1 || N < 1 || K < 1 || K > (1 << 28)) return 0;
   return mm1::gemm_workspace_bytes(M, N, K);
 }
 
@@ -646,7 +675,8 @@ int mm1_gemm(const void* x, int x_layout, long ldx, const void* w, int w_layout,
   if (!x || !w || !out) return MM1_E_NULL;
   const bool xc = x_layout == MM1_GEMM_COL, wc = w_layout == MM1_GEMM_COL;
   if ((x_layout != MM1_GEMM_ROW && !xc) || (w_layout != MM1_GEMM_ROW && !wc) || (xc && !wc)) return MM1_E_SHAPE;
-  if (M < 1 || N < 1 || K < 128 || K % 128 != 0 || N % 8 != 0 || (xc && M % 8 != 0)) return MM1_E_SHAPE;
+  if (M < 1 || N < 1 || K < 1 || K > (1 << 28) || (!xc && K % 128 != 0) || N % 8 != 0 || (xc && M % 8 != 0))
+    return MM1_E_SHAPE;
   if (w1 ? k_cut < 64 || k_cut % 64 != 0 || k_cut >= K : k_cut != 0) return MM1_E_SHAPE;
   if (out1 ? n_cut < 64 || n_cut % 64 != 0 || n_cut >= N : n_cut != 0) return MM1_E_SHAPE;
   const int w_k = w1 ? (k_cut > K - k_cut ? k_cut : K - k_cut) : K;             // longest k run in one matrix

@@ -171,7 +171,7 @@ Plan plan_of(int bn, int M, int N, int K, int n_g) {
   p.n_nblk = (N + bn - 1) / bn;
   const long total = (long)p.n_mblk * p.n_nblk;
   const int left = (int)(total % n_g);
-  const double tile = (double)(K / gemm::BK) * bn / 256, full = (double)(total / n_g);
+  const double tile = (double)gemm::windows_of(K) * bn / 256, full = (double)(total / n_g);
   const double last = left == 0 ? 0 : 2 * left <= n_g ? HALF_COST : 1;
   p.cost = (full + last) * tile;
   p.grid = gemm::persistent_grid(n_g, (int)total);
@@ -233,7 +233,7 @@ hipError_t launch_s(const Launch& l) {
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((split_sum_kernel<S, F32>), dim3(l.plan.left * 8), dim3(64 * S::TI), 0, l.stream,
                      static_cast<const float*>(l.a.workspace), l.o, l.plan.n_mblk, l.plan.n_nblk,
-                     l.plan.n_mblk * l.plan.n_nblk - l.plan.left, l.plan.left, l.a.K / gemm::BK / 2, l.plan.grid);
+                     l.plan.n_mblk * l.plan.n_nblk - l.plan.left, l.plan.left, gemm::windows_of(l.a.K) / 2, l.plan.grid);
   return hipGetLastError();
 }
 

@@ -157,9 +157,15 @@ struct Problem {
   // 64): W's part from k = k_cut on, W = [w | w1] along k.  Stride as w's.
   const __bf16* w1;
   int k_cut;
-  int K;              // reduction length, a multiple of 128
+  int K;              // reduction length, a multiple of 128 (any with both operands COL)
   int n_mblk, n_nblk;
 };
+
+// Windows of a reduction over K: whole pairs (the ring's two slots).
+__host__ __device__ inline int windows_of(int K) { return (K + 2 * BK - 1) / (2 * BK) * 2; }
+
+// Source of the copies past a ragged K.
+__device__ __attribute__((aligned(16))) static const uint32_t kZeros[4] = {0, 0, 0, 0};
 
 // The host's bound on the copies' 32-bit byte offsets from a tile's base.
 inline bool offsets_fit(Layout l, long ld, int n, int K) {
@@ -264,7 +270,8 @@ __device__ __forceinline__ void run(const Problem& p, char* smem, Pro&& pro, Epi
   constexpr int W0 = 2 * X_BYTES;                      // W's ring
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = w % S::WM, wn = w / S::WM;
-  const Tiles tiles(p.n_mblk * p.n_nblk, p.K / BK);
+  constexpr bool RAGGED_K = LX == COL && LW == COL;    // k rows past K read as zeros
+  const Tiles tiles(p.n_mblk * p.n_nblk, RAGGED_K ? windows_of(p.K) : p.K / BK);
   if (tiles.n == 0) return;
   const int n_win = tiles.windows();
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(smem));
@@ -319,21 +326,32 @@ __device__ __forceinline__ void run(const Problem& p, char* smem, Pro&& pro, Epi
     else
       return (uint32_t)(prow * (int)(2 * ld) + 2 * min(64 * n + ccol, room - 8));
   };
+  // copy n of an operand (layout, `room` rows or columns from the tile's first
+  // on, `full` of them in a tile), whose window starts at base
+  auto copy_one = [&](auto layout, int n, int room, int full, long ld, uint32_t lane, long step, const char* base,
+                      uint32_t dst) MM1_INLINE {
+    if constexpr (RAGGED_K) {
+      const int k_left = p.K - iss_kt * BK;
+      if (k_left < BK) {
+        const char* src = room >= full ? base + n * step + lane : base + edge_off(layout, n, room, ld);
+        dma16(prow < k_left ? src : reinterpret_cast<const char*>(kZeros), dst);
+        return;
+      }
+    }
+    if (room >= full) dma16_sbase(lane, base + n * step, dst);
+    else dma16_sbase(edge_off(layout, n, room, ld), base, dst);
+  };
   auto issue = [&](int slot, auto copy) MM1_INLINE {
     constexpr int C = decltype(copy)::value;
     if constexpr (C < NCX) {
-      const uint32_t dst = lds0 + slot * X_BYTES + (w + WAVES * C) * 1024;
-      if (xroom >= BM) dma16_sbase(xoff, xbase + C * xcopy, dst);
-      else dma16_sbase(edge_off(ic<LX>{}, C, xroom, p.x.ld), xbase, dst);
+      copy_one(ic<LX>{}, C, xroom, BM, p.x.ld, xoff, xcopy, xbase, lds0 + slot * X_BYTES + (w + WAVES * C) * 1024);
     } else {
       constexpr int N = C - NCX;
       const uint32_t dst = lds0 + W0 + slot * S::W_BYTES + (w + WAVES * N) * 1024;
-      if constexpr (PAIRED) {      // 128 columns of each matrix, always inside
+      if constexpr (PAIRED)        // 128 columns of each matrix, always inside
         dma16_sbase(woff, (N < 2 ? wbase : wbase1) + (N & 1) * wcopy, dst);
-      } else {
-        if (wroom >= BN) dma16_sbase(woff, wbase + N * wcopy, dst);
-        else dma16_sbase(edge_off(ic<LW>{}, N, wroom, p.w.ld), wbase, dst);
-      }
+      else
+        copy_one(ic<LW>{}, N, wroom, BN, p.w.ld, woff, wcopy, wbase, dst);
     }
   };
   auto issue_end = [&]() MM1_INLINE {

@@ -9,7 +9,8 @@
 //   FusedCrossEntropy       :193-243  loss = sum_valid (lse - target_logit) / count;
 //                                     d_logits = (softmax - onehot) * mask * grad / count
 // Layouts: hidden [T, d] bf16, weight [d, V] bf16 (the reference's
-// [d_model, vocab] matrix), targets [T] int64 (ignore_index or 0 <= t < V).
+// [d_model, vocab] matrix; LW = COL) or [V, d] (an embedding matrix as it lies
+// in memory, for a head tied to it: LW = ROW), targets [T] int64 (ignore_index or 0 <= t < V).
 //
 // Decomposition.  The logits are tiles of the persistent GEMM of gemm_core.h in
 // its single-matrix layout (256 tokens x 256 vocabulary entries per
@@ -50,13 +51,14 @@ __device__ __forceinline__ float shfl_xor32(float v) { return __shfl_xor(v, 32);
 // Bound by the GEMM core; 2.05 -> 1.63 ms at 16,384 x 1280 x 49152 (1.26
 // PFLOP/s), 125 -> 106 us at 1,000 tokens, with this core, whole-block vocabulary
 // tests instead of one per logit, and token-minor partials.
+template <gemm::Layout LW>
 __global__ __launch_bounds__(512, 1) void lm_lse_partial_kernel(
     const __bf16* __restrict__ h, const __bf16* __restrict__ w, const long long* __restrict__ targets,
     float2* __restrict__ part, float* __restrict__ tlogit, int T, int d, int V, int n_mblk, int n_nblk) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wv & 1, wn = wv >> 1, hh = lane >> 5;
-  const gemm::Problem p{{h, d, T}, {w, V, V}, w, 0, d, n_mblk, n_nblk};
+  const gemm::Problem p{{h, d, T}, {w, LW == gemm::COL ? V : d, V}, w, 0, d, n_mblk, n_nblk};
   // the gathered column of each of the lane's tokens, loaded at the tile's
   // first window (the loads land during the products)
   int tcol[4];
@@ -67,7 +69,7 @@ __global__ __launch_bounds__(512, 1) void lm_lse_partial_kernel(
       tcol[i] = t < 0 || t >= V ? 0 : (int)t;     // the reference gathers column clamp(t, min=0)
     }
   };
-  gemm::run<gemm::ROW, gemm::COL, false, gemm::Wide256, gemm::WholeTiles>(p, smem, pro, [&](int mb, int nb, f32x16 (&acc)[2][4], int) MM1_INLINE {
+  gemm::run<gemm::ROW, LW, false, gemm::Wide256, gemm::WholeTiles>(p, smem, pro, [&](int mb, int nb, f32x16 (&acc)[2][4], int) MM1_INLINE {
     const int v0 = nb * 256 + 64 * wn;             // this wave's 64 vocabulary entries
     const bool inside = v0 < V;
 #pragma unroll
@@ -166,11 +168,11 @@ __global__ __launch_bounds__(COMBINE_THREADS) void lm_lse_combine_kernel(
   }
 }
 
-// d_logits of vocabulary entries [v0, v0 + vn): the GEMM runs over the
-// columns of weight + v0; out[t][v] (row stride ld) = bf16((exp(l - lse[t]) -
+// d_logits of vocabulary entries [v0, v0 + vn): the GEMM runs over those
+// columns (or rows) of weight; out[t][v] (row stride ld) = bf16((exp(l - lse[t]) -
 // [v0 + v == target[t]]) * scale) for valid targets, 0 for ignored ones.
 // `scale` is a device scalar (the loss gradient over the valid count).
-template <bool NT>
+template <gemm::Layout LW, bool NT>
 __global__ __launch_bounds__(512, 1) void lm_dlogits_kernel(
     const __bf16* __restrict__ h, const __bf16* __restrict__ w, const long long* __restrict__ targets,
     const float* __restrict__ lse, const float* __restrict__ scale, __bf16* __restrict__ out, long ld,
@@ -178,7 +180,8 @@ __global__ __launch_bounds__(512, 1) void lm_dlogits_kernel(
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wv & 1, wn = wv >> 1;
-  const gemm::Problem p{{h, d, T}, {w + v0, V, vn}, w, 0, d, n_mblk, n_nblk};
+  const __bf16* wv0 = w + (LW == gemm::COL ? (long)v0 : (long)v0 * d);
+  const gemm::Problem p{{h, d, T}, {wv0, LW == gemm::COL ? V : d, vn}, wv0, 0, d, n_mblk, n_nblk};
   const float sc = *scale;
   // the rows go out through 4 KiB per wave above the GEMM's ring
   char* stage = smem + gemm::Wide256::RING + gemm::Wide256::STAGE_BYTES * wv;
@@ -198,7 +201,7 @@ __global__ __launch_bounds__(512, 1) void lm_dlogits_kernel(
       l2[i] = lse[tok] * kLog2e;
     }
   };
-  gemm::run<gemm::ROW, gemm::COL, false, gemm::Wide256, gemm::WholeTiles>(p, smem, pro, [&](int mb, int nb, f32x16 (&acc)[2][4], int) MM1_INLINE {
+  gemm::run<gemm::ROW, LW, false, gemm::Wide256, gemm::WholeTiles>(p, smem, pro, [&](int mb, int nb, f32x16 (&acc)[2][4], int) MM1_INLINE {
     const int c0 = nb * 256 + 64 * wn;             // this wave's first column of the chunk
     const long tok0 = (long)mb * gemm::BM + 128 * wm;
     // the target's column among the wave's 64, counted from the lane's first;
@@ -246,21 +249,21 @@ size_t lm_head_workspace_bytes(int T, int V) {
   return (size_t)T * n_part * sizeof(float2) + (size_t)T * sizeof(float) + 256;
 }
 
-hipError_t launch_lm_lse(const void* hidden, const void* weight, const long long* targets, long long ignore_index,
+hipError_t launch_lm_lse(const void* hidden, const void* weight, bool vocab_rows, const long long* targets, long long ignore_index,
                          float* lse, float* tlogit_out, float* loss, void* workspace, int T, int d, int V,
                          hipStream_t stream) {
   int n_mblk, n_nblk, grid;
   hipError_t e = gemm_geometry(T, V, n_mblk, n_nblk, grid);
   if (e != hipSuccess) return e;
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(lm_lse_partial_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm::Wide256::RING);
+  auto kern = vocab_rows ? lm_lse_partial_kernel<gemm::ROW> : lm_lse_partial_kernel<gemm::COL>;
+  e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm::Wide256::RING);
   if (e != hipSuccess) return e;
   const int n_part = 4 * n_nblk;
   auto part = static_cast<float2*>(workspace);
   float* tl = tlogit_out != nullptr
                   ? tlogit_out
                   : reinterpret_cast<float*>(static_cast<char*>(workspace) + (size_t)T * n_part * sizeof(float2));
-  hipLaunchKernelGGL(lm_lse_partial_kernel, dim3(grid), dim3(512), gemm::Wide256::RING, stream,
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), gemm::Wide256::RING, stream,
                      static_cast<const __bf16*>(hidden), static_cast<const __bf16*>(weight), targets, part, tl,
                      T, d, V, n_mblk, n_nblk);
   hipLaunchKernelGGL(lm_lse_combine_kernel, dim3((T + COMBINE_TOKENS - 1) / COMBINE_TOKENS), dim3(COMBINE_THREADS), 0, stream, part, tl, targets, lse,
@@ -268,7 +271,7 @@ hipError_t launch_lm_lse(const void* hidden, const void* weight, const long long
   return hipGetLastError();
 }
 
-hipError_t launch_lm_dlogits(const void* hidden, const void* weight, const long long* targets,
+hipError_t launch_lm_dlogits(const void* hidden, const void* weight, bool vocab_rows, const long long* targets,
                              long long ignore_index, const float* lse, const float* scale, void* dlogits, long ld,
                              int T, int d, int V, int v0, int vn, hipStream_t stream) {
   int n_mblk, n_nblk, grid;
@@ -279,7 +282,9 @@ hipError_t launch_lm_dlogits(const void* hidden, const void* weight, const long 
   // stores (16,384 tokens, whole vocabulary: 2.03 -> 1.75 ms with the
   // core of gemm_core.h); at 1,000 tokens (98 MB) the product that reads them next is 28 us
   // faster when they were stored through the caches.
-  auto kern = (long)T * vn * 2 > gemm::CACHED_BYTES ? lm_dlogits_kernel<true> : lm_dlogits_kernel<false>;
+  const bool nt = (long)T * vn * 2 > gemm::CACHED_BYTES;
+  auto kern = vocab_rows ? (nt ? lm_dlogits_kernel<gemm::ROW, true> : lm_dlogits_kernel<gemm::ROW, false>)
+                         : (nt ? lm_dlogits_kernel<gemm::COL, true> : lm_dlogits_kernel<gemm::COL, false>);
   e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, stream,

@@ -30,8 +30,8 @@ def _layout(t):
 
 
 def applies(x, w) -> bool:
-    """Whether mm1_gemm takes x [M, K] w [N, K]^T (K a multiple of 128, N of
-    8, not x k-major with w k-contiguous) and was measured faster than
+    """Whether mm1_gemm takes x [M, K] w [N, K]^T (K a multiple of 128 unless
+    both are k-major, N of 8, not x k-major with w k-contiguous) and was measured faster than
     hipBLASLt's GEMM at such a size (MI355X; T tokens, widths 1280 to 49152):
 
     * with w k-major from M N K = 2.4e10 on: x k-major (weight gradients)
@@ -49,14 +49,14 @@ def applies(x, w) -> bool:
         return False
     m, k = x.shape
     n = w.shape[0]
-    if k % 128 or n % 8 or m < 1 or w.shape[1] != k or w.device != x.device:
+    if (k % 128 and lx[0] == ROW) or n % 8 or m < 1 or k < 1 or w.shape[1] != k or w.device != x.device:
         return False
     for (layout, ld), rows in ((lx, m), (lw, n)):
         if (256 * ld + k if layout == ROW else 64 * ld + rows) >= 1 << 30 or rows > 1 << 26:
             return False
     if lw[0] == COL:
         return m * n * k >= 24 * 10 ** 9
-    return (n % 320 == 0 and m * n >= 230 * 256 * 320) or (k >= 16384 and m * n >= 20 * 256 * 256)
+    return (n % 320 == 0 and m * n >= 230 * 256 * 320) or (k >= 16384 and m * n >= 16 * 256 * 256)
 
 
 def applies_joined(x, w, w1) -> bool:

@@ -87,7 +87,17 @@ class LseKernel:
         T, d, V = self.shape
         _require(hidden, "hidden", (T, d))
         _require(weight, "weight", (d, V))
-        lib = _lib.load()
+        return self._forward(_lib.load().mm1_lm_head_lse, hidden, weight, targets, ignore_index)
+
+    def forward_rows(self, hidden, weight, targets=None, ignore_index=IGNORE_INDEX):
+        """forward() with the weight stored [V, d]."""
+        T, d, V = self.shape
+        _require(hidden, "hidden", (T, d))
+        _require(weight, "weight", (V, d))
+        return self._forward(_lib.load().mm1_lm_head_lse_rows, hidden, weight, targets, ignore_index)
+
+    def _forward(self, entry, hidden, weight, targets, ignore_index):
+        T, d, V = self.shape
         dev = hidden.device
         lse = torch.empty(T, dtype=torch.float32, device=dev)
         tl = loss = None
@@ -95,12 +105,11 @@ class LseKernel:
             _require(targets, "targets", (T,), torch.int64)
             tl = torch.empty(T, dtype=torch.float32, device=dev)
             loss = torch.empty(T, dtype=torch.float32, device=dev)
-        ws_bytes = lib.mm1_lm_head_workspace_size(T, V)
+        ws_bytes = _lib.load().mm1_lm_head_workspace_size(T, V)
         ws = torch.empty(ws_bytes // 4 + 1, dtype=torch.float32, device=dev)
         ptr = lambda t: None if t is None else t.data_ptr()
-        rc = lib.mm1_lm_head_lse(hidden.data_ptr(), weight.data_ptr(), ptr(targets), int(ignore_index),
-                                 lse.data_ptr(), ptr(tl), ptr(loss), ws.data_ptr(), ws_bytes, T, d, V,
-                                 _stream(dev))
+        rc = entry(hidden.data_ptr(), weight.data_ptr(), ptr(targets), int(ignore_index), lse.data_ptr(), ptr(tl),
+                   ptr(loss), ws.data_ptr(), ws_bytes, T, d, V, _stream(dev))
         _lib.check(rc, "mm1_lm_head_lse")
         return lse, tl, loss
 
@@ -109,13 +118,20 @@ class LseKernel:
 
     def dlogits(self, hidden, weight, targets, lse, scale, v0, vn, out=None, ignore_index=IGNORE_INDEX):
         """bf16 d_logits of vocabulary entries [v0, v0 + vn) into out [T, vn]."""
+        return self._dlogits(_lib.load().mm1_lm_head_dlogits, hidden, weight, targets, lse, scale, v0, vn, out,
+                             ignore_index)
+
+    def dlogits_rows(self, hidden, weight, targets, lse, scale, v0, vn, out=None, ignore_index=IGNORE_INDEX):
+        """dlogits() with the weight stored [V, d]."""
+        return self._dlogits(_lib.load().mm1_lm_head_dlogits_rows, hidden, weight, targets, lse, scale, v0, vn, out,
+                             ignore_index)
+
+    def _dlogits(self, entry, hidden, weight, targets, lse, scale, v0, vn, out, ignore_index):
         T, d, V = self.shape
         if out is None:
             out = torch.empty(T, vn, dtype=DTYPE, device=hidden.device)
-        rc = _lib.load().mm1_lm_head_dlogits(hidden.data_ptr(), weight.data_ptr(), targets.data_ptr(),
-                                             int(ignore_index), lse.data_ptr(), scale.data_ptr(),
-                                             out.data_ptr(), out.stride(0), T, d, V, v0, vn,
-                                             _stream(hidden.device))
+        rc = entry(hidden.data_ptr(), weight.data_ptr(), targets.data_ptr(), int(ignore_index), lse.data_ptr(),
+                   scale.data_ptr(), out.data_ptr(), out.stride(0), T, d, V, v0, vn, _stream(hidden.device))
         _lib.check(rc, "mm1_lm_head_dlogits")
         return out
 
@@ -157,9 +173,27 @@ def gather_target_logits(hidden, weight, targets):
     return (hidden.to(acc) * rows.to(acc)).sum(-1)
 
 
-def _matmul(x, w):
+def _matmul(x, w, out_dtype=DTYPE):
     """x w^T on the GEMM core where it applies (gemm.py), else torch's GEMM."""
-    return gemm.product(x, w) if gemm.applies(x, w) else x @ w.t()
+    if gemm.applies(x, w):
+        return gemm.product(x, w, out_dtype=out_dtype)
+    return x @ w.t() if out_dtype == DTYPE else torch.mm(x, w.t(), out_dtype=out_dtype)
+
+
+def _check_bf16_hip(hidden, weight):
+    if not (hidden.is_cuda and hidden.dtype is DTYPE and weight.dtype is DTYPE):
+        raise ValueError("fused_cross_entropy runs the HIP kernels: hidden and weight must be bf16 "
+                         f"HIP tensors (got {hidden.dtype} on {hidden.device}, {weight.dtype})")
+
+
+def _mean_loss(per_token, targets):
+    """(mean over the tokens that are not IGNORE_INDEX, their count, at least 1)."""
+    count = (targets != IGNORE_INDEX).sum().clamp(min=1)
+    return per_token.sum() / count, count
+
+
+def _chunk_size(chunk, vocab):
+    return max(128, (min(chunk, vocab) // 128) * 128)
 
 
 class FusedCrossEntropy(torch.autograd.Function):
@@ -171,14 +205,11 @@ class FusedCrossEntropy(torch.autograd.Function):
     def forward(ctx, hidden, weight, targets, chunk):
         tokens, d_model = hidden.shape
         vocab = weight.shape[1]
-        if not (hidden.is_cuda and hidden.dtype is DTYPE and weight.dtype is DTYPE):
-            raise ValueError("fused_cross_entropy runs the HIP kernels: hidden and weight must be bf16 "
-                             f"HIP tensors (got {hidden.dtype} on {hidden.device}, {weight.dtype})")
+        _check_bf16_hip(hidden, weight)
         kernel = get_kernel((tokens, d_model, vocab))
         targets = targets.contiguous()
         lse, _, per_token = kernel.forward(hidden, weight, targets)
-        count = (targets != IGNORE_INDEX).sum().clamp(min=1)
-        loss = per_token.sum() / count
+        loss, count = _mean_loss(per_token, targets)
         ctx.save_for_backward(hidden, weight, targets, lse, count)
         ctx.chunk = chunk
         return loss
@@ -188,7 +219,7 @@ class FusedCrossEntropy(torch.autograd.Function):
         hidden, weight, targets, lse, count = ctx.saved_tensors
         tokens, d_model = hidden.shape
         vocab = weight.shape[1]
-        chunk = max(128, (min(ctx.chunk, vocab) // 128) * 128)
+        chunk = _chunk_size(ctx.chunk, vocab)
         kernel = get_kernel((tokens, d_model, vocab))
         scale = (grad_loss.float() / count).reshape(1).contiguous()
         if chunk >= vocab:
@@ -202,6 +233,50 @@ class FusedCrossEntropy(torch.autograd.Function):
             dl = kernel.dlogits(hidden, weight, targets, lse, scale, start, stop - start)
             d_hidden += _matmul(dl, weight[:, start:stop]).float()
             d_weight[:, start:stop] = _matmul(hidden.t(), dl.t())
+        return d_hidden.to(hidden.dtype), d_weight, None, None
+
+
+class TiedCrossEntropy(torch.autograd.Function):
+    """FusedCrossEntropy for a head tied to its embedding: `embedding` is the
+    [V, d] matrix as it lies in memory, which the kernels read by rows, so no
+    transposed copy is made (at V 49152, d 1280 the transpose alone took 255
+    us), and its gradient leaves the product in the embedding's own layout and
+    dtype (fp32 sums, rounded once or not at all)."""
+
+    @staticmethod
+    def forward(ctx, hidden, embedding, targets, chunk):
+        tokens, d_model = hidden.shape
+        vocab = embedding.shape[0]
+        weight = embedding.to(DTYPE).contiguous()
+        _check_bf16_hip(hidden, weight)
+        kernel = get_kernel((tokens, d_model, vocab))
+        targets = targets.contiguous()
+        lse, _, per_token = kernel.forward_rows(hidden, weight, targets)
+        loss, count = _mean_loss(per_token, targets)
+        ctx.save_for_backward(hidden, weight, targets, lse, count)
+        ctx.chunk, ctx.grad_dtype = chunk, embedding.dtype
+        return loss
+
+    @staticmethod
+    def backward(ctx, grad_loss):
+        hidden, weight, targets, lse, count = ctx.saved_tensors
+        tokens, d_model = hidden.shape
+        vocab = weight.shape[0]
+        chunk = _chunk_size(ctx.chunk, vocab)
+        kernel = get_kernel((tokens, d_model, vocab))
+        scale = (grad_loss.float() / count).reshape(1).contiguous()
+        wide = torch.float32 if ctx.grad_dtype == torch.float32 else DTYPE
+        if chunk >= vocab:
+            dl = kernel.dlogits_rows(hidden, weight, targets, lse, scale, 0, vocab)
+            d_weight = _matmul(dl.t(), hidden.t(), wide).to(ctx.grad_dtype) if ctx.needs_input_grad[1] else None
+            return _matmul(dl, weight.t()), d_weight, None, None
+        d_weight = torch.empty(vocab, d_model, dtype=ctx.grad_dtype, device=hidden.device)
+        d_hidden = torch.zeros(tokens, d_model, dtype=torch.float32, device=hidden.device)
+        for start in range(0, vocab, chunk):
+            stop = min(start + chunk, vocab)
+            dl = kernel.dlogits_rows(hidden, weight, targets, lse, scale, start, stop - start)
+            d_hidden += _matmul(dl, weight[start:stop].t()).float()
+            d_weight[start:stop] = _matmul(dl.t(), hidden.t(), wide)
         return d_hidden.to(hidden.dtype), d_weight, None, None
 
 
@@ -253,8 +328,11 @@ class LMHead(nn.Module):
         return self.embedding[0].weight.t() if self.cfg.tied else self.weight
 
     def _loss_hip(self, rows, weight, targets):
-        # bf16 kernels: the fp32 stream and the tied matrix's transposed view
-        # become contiguous bf16 here (LM:313-323)
+        # bf16 kernels: the fp32 stream and matrix become contiguous bf16 here
+        # (LM:313-323); a tied matrix is read in the embedding's own layout
+        if self.cfg.tied:
+            return TiedCrossEntropy.apply(rows.to(DTYPE).contiguous(), self.embedding[0].weight, targets,
+                                          self.cfg.chunk)
         return fused_cross_entropy(rows.to(DTYPE).contiguous(), weight.to(DTYPE).contiguous(), targets,
                                    self.cfg.chunk)
 

@@ -61,12 +61,24 @@ def test_joined_weights_and_split_output(hip_device, T, d, F):
     d_gu = operand(T, 2 * F, False, gen, hip_device)
     wg, wu = (operand(d, F, False, gen, hip_device) for _ in range(2))
     check(gemm.product(d_gu, wg, w1=wu), d_gu, torch.cat((wg, wu), dim=1))
-    if T % 128:
-        return
     x = operand(d, T, True, gen, hip_device)
     lo, hi = gemm.product(x, d_gu.t(), split=F)
     check(lo, x, d_gu.t()[:F])
     check(hi, x, d_gu.t()[F:])
+
+
+@pytest.mark.parametrize("K", [1, 7, 63, 64, 65, 127, 129, 1000, 4099, 16383])
+def test_ragged_reduction_of_weight_gradients(hip_device, K):
+    """Both operands k-major: the k rows past K, which memory may hold NaN at,
+    count as zeros."""
+    gen = torch.Generator(device=hip_device).manual_seed(K)
+    for M, N in ((264, 1288), (1280, 640)):
+        xs, ws = (torch.full((K + 130, n), float("nan"), dtype=torch.bfloat16, device=hip_device) for n in (M, N))
+        for t in (xs, ws):
+            t[:K] = torch.randn(K, t.shape[1], device=hip_device, generator=gen).to(torch.bfloat16)
+        x, w = xs[:K].t(), ws[:K].t()
+        for dtype in (torch.bfloat16, torch.float32):
+            check(gemm.product(x, w, out_dtype=dtype), x, w)
 
 
 def test_c_abi_refuses_what_the_kernels_do_not_take(hip_device):

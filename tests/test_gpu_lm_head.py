@@ -131,3 +131,26 @@ def test_fused_cross_entropy_deterministic(hip_device):
         runs.append((loss.item(), hd.grad.cpu(), wd.grad.cpu()))
     assert runs[0][0] == runs[1][0]
     assert torch.equal(runs[0][1], runs[1][1]) and torch.equal(runs[0][2], runs[1][2])
+
+
+@pytest.mark.parametrize("T,V,chunk,dtype", [(300, 49152, 49152, torch.float32), (1, 128, 128, torch.float32),
+                                             (333, 1280, 256, torch.float32), (257, 2048, 2048, torch.bfloat16)])
+def test_tied_head_reads_the_embedding_by_rows(hip_device, T, V, chunk, dtype):
+    """A head tied to its embedding matrix [V, d] against the same loss on a
+    transposed copy: the loss and d_hidden agree to the order of fp32 sums, and
+    the embedding's gradient to its one bf16 rounding on top."""
+    from mimansm1_v1_amd import lm_head as L
+    h, w, t = (x.to(hip_device) for x in LMO.make_inputs(T, 1280, V, seed=T, n_ignore=T // 8))
+    emb = torch.nn.Embedding(V, 1280, device=hip_device, dtype=dtype, _weight=w.t().contiguous().to(dtype))
+    head = L.LMHead(L.HeadConfig(vocab=V, logit_scale=1.0, chunk=chunk), emb)
+    rows, wd = h.clone().requires_grad_(True), w.to(torch.bfloat16).requires_grad_(True)
+    hid = h.clone().requires_grad_(True)
+    loss = head(hid, t)
+    want = L.fused_cross_entropy(rows, wd, t, chunk)
+    loss.backward()
+    want.backward()
+    assert abs(loss.item() - want.item()) <= 1e-5 * abs(want.item())
+    assert emb.weight.grad.dtype == dtype and hid.grad.dtype == h.dtype
+    for a, b in ((hid.grad, rows.grad), (emb.weight.grad, wd.grad.t())):
+        a, b = a.double(), b.double()
+        assert (a - b).norm() <= 2.0 ** -8 * b.norm()
