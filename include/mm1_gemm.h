@@ -46,6 +46,12 @@ int mm1_gemm(const void* x, int x_layout, long ldx, const void* w, int w_layout,
              int k_cut, void* out, void* out1, int n_cut, long ldo, int out_f32, void* workspace,
              size_t workspace_bytes, int M, int N, int K, void* stream);
 
+/* dst = the fp32 tensors src0 .. src3 rounded to bf16 (nearest even), one
+ * after the other (n0 .. n3 values, each a multiple of 8, 0 for none): the
+ * operands of a product whose activations and weights are held in fp32. */
+int mm1_cast_bf16(const float* src0, long n0, const float* src1, long n1, const float* src2, long n2,
+                  const float* src3, long n3, void* dst, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -64,6 +64,7 @@ SIGNATURES = {
     "mm1_gemm_workspace_size": (_c_size, [_c_int, _c_int, _c_int]),
     "mm1_gemm": (_c_int, [_vp, _c_int, ctypes.c_long, _vp, _c_int, ctypes.c_long, _vp, _c_int, _vp, _vp, _c_int,
                           ctypes.c_long, _c_int, _vp, _c_size, _c_int, _c_int, _c_int, _vp]),
+    "mm1_cast_bf16": (_c_int, [_vp, ctypes.c_long] * 4 + [_vp, _vp]),
     "mm1_attn_strerror": (ctypes.c_char_p, [_c_int]),
 }
 

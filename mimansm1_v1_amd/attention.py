@@ -119,7 +119,7 @@ BWD_TILES = dict(dkdv_block_M=128, dkdv_block_N=32, dkdv_waves=8, dkdv_stages=7,
 # ---------------------------------------------------------------------------
 # Kernel handles
 def _stream(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)   # torch.cuda.current_stream costs 2 us a call
 
 
 # True: the backward runs its dQ launch on a second stream of the device,
@@ -145,6 +145,8 @@ def _side_stream(device) -> "torch.cuda.Stream":
 def _require(t: torch.Tensor, name: str, shape, dtype=DTYPE):
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
+    if t.is_cuda and t.dtype is dtype and t.shape == shape and t.is_contiguous():
+        return
     if not t.is_cuda:
         raise ValueError(f"{name} must be a CUDA (HIP) tensor, got device {t.device}")
     if t.dtype != dtype:
@@ -169,7 +171,14 @@ class _Kernel:
         self.causal, self.groups = bool(causal), groups
         self.kv_heads = heads // groups
         self.sm_scale = (1.0 / dim) ** 0.5
-        _lib.load()
+        self.q_shape, self.kv_shape = (batch, seq_len, heads, dim), (batch, seq_len, self.kv_heads, dim)
+        self.lse_shape = (batch, heads, seq_len)
+        # what the C calls take besides the pointers, built once per handle
+        self.c_shape = (batch, seq_len, heads, self.kv_heads, dim)
+        self.c_args = (*self.c_shape, int(self.causal), self.sm_scale)
+        lib = _lib.load()
+        self.state_bytes = lib.mm1_attn_fwd_state_size(*self.c_shape)
+        self.ws_bytes = lib.mm1_attn_bwd_workspace_size(*self.c_shape)
         self.tiles = tile_index(self.kind, self.config)
         if self.tiles is None:
             raise ValueError(f"{self.kind} config {self.config} is not a tiling compiled into "
@@ -179,11 +188,6 @@ class _Kernel:
         return f"<{type(self).__name__} shape={self.shape} config={self.config}>"
 
 
-def _state(lib, B, S, H, Hkv, D, device):
-    """A forward state buffer (mm1_attn_fwd_state_size bytes, uint8)."""
-    return torch.empty(lib.mm1_attn_fwd_state_size(B, S, H, Hkv, D), dtype=torch.uint8, device=device)
-
-
 class FwdKernel(_Kernel):
     """(q, k, v) -> (O, lse2); replaces flash_fwd (AT:110-190).  ``run``
     also returns the forward state the backward reads (the fp16 operand
@@ -191,17 +195,16 @@ class FwdKernel(_Kernel):
     kind = "fwd"
 
     def run(self, q, k, v):
-        B, H, S, D, Hkv = self.batch, self.heads, self.seq_len, self.dim, self.kv_heads
-        _require(q, "q", (B, S, H, D))
-        _require(k, "k", (B, S, Hkv, D))
-        _require(v, "v", (B, S, Hkv, D))
-        lib = _lib.load()
+        _require(q, "q", self.q_shape)
+        _require(k, "k", self.kv_shape)
+        _require(v, "v", self.kv_shape)
+        device = q.device
         out = torch.empty_like(q)
-        lse = torch.empty(B, H, S, dtype=torch.float32, device=q.device)
-        state = _state(lib, B, S, H, Hkv, D, q.device)
-        rc = lib.mm1_attn_fwd_tiles(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
-                                    state.data_ptr(), state.numel(), B, S, H, Hkv, D, int(self.causal),
-                                    self.sm_scale, self.tiles, _stream(q.device))
+        lse = torch.empty(self.lse_shape, dtype=torch.float32, device=device)
+        state = torch.empty(self.state_bytes, dtype=torch.uint8, device=device)
+        rc = _lib.load().mm1_attn_fwd_tiles(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                            lse.data_ptr(), state.data_ptr(), self.state_bytes, *self.c_args,
+                                            self.tiles, _stream(device))
         _lib.check(rc, "mm1_attn_fwd_tiles")
         return out, lse, state
 
@@ -221,54 +224,53 @@ class BwdKernel(_Kernel):
     kind = "bwd"
 
     def _check_grads(self, dq, dk, dv):
-        B, H, S, D, Hkv = self.batch, self.heads, self.seq_len, self.dim, self.kv_heads
-        _require(dq, "dq", (B, S, H, D))
-        _require(dk, "dk", (B, S, Hkv, D))
-        _require(dv, "dv", (B, S, Hkv, D))
+        _require(dq, "dq", self.q_shape)
+        _require(dk, "dk", self.kv_shape)
+        _require(dv, "dv", self.kv_shape)
 
     def __call__(self, q, k, v, grad_out, lse, delta, dq, dk, dv):
-        B, H, S, D, Hkv = self.batch, self.heads, self.seq_len, self.dim, self.kv_heads
-        _require(q, "q", (B, S, H, D))
-        _require(k, "k", (B, S, Hkv, D))
-        _require(v, "v", (B, S, Hkv, D))
-        _require(grad_out, "grad_out", (B, S, H, D))
-        _require(lse, "lse", (B, H, S), torch.float32)
-        _require(delta, "delta", (B, H, S), torch.float32)
+        _require(q, "q", self.q_shape)
+        _require(k, "k", self.kv_shape)
+        _require(v, "v", self.kv_shape)
+        _require(grad_out, "grad_out", self.q_shape)
+        _require(lse, "lse", self.lse_shape, torch.float32)
+        _require(delta, "delta", self.lse_shape, torch.float32)
         self._check_grads(dq, dk, dv)
         lib = _lib.load()
-        state = _state(lib, B, S, H, Hkv, D, q.device)
+        state = torch.empty(self.state_bytes, dtype=torch.uint8, device=q.device)
         rc = lib.mm1_attn_prep(q.data_ptr(), k.data_ptr(), v.data_ptr(), state.data_ptr(), state.numel(),
-                               B, S, H, Hkv, D, _stream(q.device))
+                               *self.c_shape, _stream(q.device))
         _lib.check(rc, "mm1_attn_prep")
-        ws = self._workspace(lib, q.device)
+        ws = torch.empty(self.ws_bytes, dtype=torch.uint8, device=q.device)
         rc = lib.mm1_attn_bwd_prep_delta(grad_out.data_ptr(), delta.data_ptr(), lse.data_ptr(), state.data_ptr(),
-                                         state.numel(), ws.data_ptr(), ws.numel(), B, S, H, Hkv, D, self.sm_scale,
+                                         state.numel(), ws.data_ptr(), ws.numel(), *self.c_shape, self.sm_scale,
                                          _stream(q.device))
         _lib.check(rc, "mm1_attn_bwd_prep_delta")
         self._stages(lib, state, ws, dq, dk, dv)
 
     def run_saved(self, out, grad_out, lse, state, dq, dk, dv):
         """dQ, dK, dV from the forward's (out, lse, state) and dO."""
-        B, H, S, D, Hkv = self.batch, self.heads, self.seq_len, self.dim, self.kv_heads
-        _require(out, "out", (B, S, H, D))
-        _require(grad_out, "grad_out", (B, S, H, D))
-        _require(lse, "lse", (B, H, S), torch.float32)
+        _require(out, "out", self.q_shape)
+        _require(grad_out, "grad_out", self.q_shape)
+        _require(lse, "lse", self.lse_shape, torch.float32)
         self._check_grads(dq, dk, dv)
         lib = _lib.load()
-        ws = self._workspace(lib, out.device)
+        device = out.device
+        ws = torch.empty(self.ws_bytes, dtype=torch.uint8, device=device)
+        if not self.config.get("overlap_dq", OVERLAP_DQ):       # every stage on one stream: one call
+            rc = lib.mm1_attn_bwd_tiles(out.data_ptr(), grad_out.data_ptr(), lse.data_ptr(), state.data_ptr(),
+                                        state.numel(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(),
+                                        self.ws_bytes, *self.c_args, *self.tiles, _stream(device))
+            _lib.check(rc, "mm1_attn_bwd_tiles")
+            return
         rc = lib.mm1_attn_bwd_prep(out.data_ptr(), grad_out.data_ptr(), lse.data_ptr(), state.data_ptr(),
-                                   state.numel(), ws.data_ptr(), ws.numel(), B, S, H, Hkv, D, self.sm_scale,
-                                   _stream(out.device))
+                                   state.numel(), ws.data_ptr(), ws.numel(), *self.c_shape, self.sm_scale,
+                                   _stream(device))
         _lib.check(rc, "mm1_attn_bwd_prep")
         self._stages(lib, state, ws, dq, dk, dv)
 
-    def _workspace(self, lib, device):
-        B, H, S, D, Hkv = self.batch, self.heads, self.seq_len, self.dim, self.kv_heads
-        return torch.empty(lib.mm1_attn_bwd_workspace_size(B, S, H, Hkv, D), dtype=torch.uint8, device=device)
-
     def _stages(self, lib, state, ws, dq, dk, dv):
-        B, H, S, D, Hkv = self.batch, self.heads, self.seq_len, self.dim, self.kv_heads
-        shape = (B, S, H, Hkv, D, int(self.causal), self.sm_scale)
+        shape = self.c_args
         dkdv_tiles, dq_tiles = self.tiles
         st, wsp = (state.data_ptr(), state.numel()), (ws.data_ptr(), ws.numel())
         if not self.config.get("overlap_dq", OVERLAP_DQ):
@@ -290,7 +292,7 @@ class BwdKernel(_Kernel):
             rc = lib.mm1_attn_bwd_dkdv_tiles(*st, dk.data_ptr(), dv.data_ptr(), *wsp, *shape, dkdv_tiles,
                                              main.cuda_stream)
             _lib.check(rc, "mm1_attn_bwd_dkdv_tiles")
-            rc = lib.mm1_attn_bwd_dkdv_reduce_tiles(*wsp, dk.data_ptr(), dv.data_ptr(), B, S, H, Hkv, D,
+            rc = lib.mm1_attn_bwd_dkdv_reduce_tiles(*wsp, dk.data_ptr(), dv.data_ptr(), *self.c_shape,
                                                     int(self.causal), dkdv_tiles, main.cuda_stream)
             _lib.check(rc, "mm1_attn_bwd_dkdv_reduce_tiles")
         finally:
@@ -582,24 +584,67 @@ class BF16Linear(torch.autograd.Function):
         xb, wb = x.to(DTYPE), w.to(DTYPE)
         ctx.save_for_backward(xb, wb)
         ctx.x_dtype, ctx.w_dtype = x.dtype, w.dtype
-        x2 = xb.reshape(-1, xb.shape[-1])
-        if gemm.applies(x2, wb):
-            return gemm.product(x2, wb).reshape(*xb.shape[:-1], wb.shape[0])
-        return F.linear(xb, wb)
+        return _linear(xb, wb)
 
     @staticmethod
     def backward(ctx, dy):
-        xb, wb = ctx.saved_tensors
-        n, k = wb.shape
-        dy2 = dy.reshape(-1, n).to(DTYPE)
-        x2 = xb.reshape(-1, k)
-        dx = dw = None
-        if ctx.needs_input_grad[0]:
-            dx = gemm.product(dy2, wb.t()) if gemm.applies(dy2, wb.t()) else dy2 @ wb
-            dx = dx.reshape(*dy.shape[:-1], k).to(ctx.x_dtype)
-        if ctx.needs_input_grad[1]:
-            dw = wgrad(dy2, x2, PROJ_DW_CHUNKS).to(ctx.w_dtype)
-        return dx, dw
+        return _linear_grads(ctx, dy)
+
+
+def _linear(xb, wb):
+    x2 = xb.reshape(-1, xb.shape[-1])
+    if gemm.applies(x2, wb):
+        return gemm.product(x2, wb).reshape(*xb.shape[:-1], wb.shape[0])
+    return F.linear(xb, wb)
+
+
+def _linear_grads(ctx, dy):
+    """(dX, dW) of _linear for the inputs that need them; dW in fp32's sums,
+    one rounding to the weight's dtype."""
+    xb, wb = ctx.saved_tensors
+    n, k = wb.shape
+    dy2 = dy.reshape(-1, n).to(DTYPE)
+    dx = dw = None
+    if ctx.needs_input_grad[0]:
+        dx = gemm.product(dy2, wb.t()) if gemm.applies(dy2, wb.t()) else dy2 @ wb
+        dx = dx.reshape(*dy.shape[:-1], k).to(ctx.x_dtype)
+    if any(ctx.needs_input_grad[1:]):
+        dw = wgrad(dy2, xb.reshape(-1, k), PROJ_DW_CHUNKS).to(ctx.w_dtype)
+    return dx, dw
+
+
+class QKVLinear(torch.autograd.Function):
+    """BF16Linear against wq | wk | wv: one product, whose bf16 operands one
+    cast launch writes from the fp32 parameters (and an fp32 x) into one
+    buffer; the parameters' gradients are row blocks of the one dW."""
+
+    @staticmethod
+    def forward(ctx, x, wq, wk, wv):
+        rows = tuple(w.shape[0] for w in (wq, wk, wv))
+        k = wq.shape[1]
+        with_x = _castable(x)
+        buf = torch.empty((x.numel() if with_x else 0) + sum(rows) * k, dtype=DTYPE, device=x.device)
+        first = x.numel() if with_x else 0
+        rc = _lib.load().mm1_cast_bf16(x.data_ptr() if with_x else None, first, wq.data_ptr(), wq.numel(),
+                                       wk.data_ptr(), wk.numel(), wv.data_ptr(), wv.numel(), buf.data_ptr(),
+                                       _stream(x.device))
+        _lib.check(rc, "mm1_cast_bf16")
+        xb = buf[:first].view(x.shape) if with_x else x.to(DTYPE)
+        wb = buf[first:].view(sum(rows), k)
+        ctx.save_for_backward(xb, wb)
+        ctx.x_dtype, ctx.w_dtype, ctx.rows = x.dtype, wq.dtype, rows
+        return _linear(xb, wb)
+
+    @staticmethod
+    def backward(ctx, dy):
+        dx, dw = _linear_grads(ctx, dy)
+        return dx, *(dw.split(ctx.rows) if dw is not None else (None,) * 3)
+
+
+def _castable(t) -> bool:
+    """What mm1_cast_bf16 reads: fp32, contiguous, whole 16-byte pieces."""
+    return (t.is_cuda and t.dtype is torch.float32 and t.is_contiguous() and t.numel() % 8 == 0 and t.numel() > 0
+            and t.data_ptr() % 16 == 0)
 
 
 def _autocast_bf16() -> bool:
@@ -635,8 +680,8 @@ class QKNormRope(torch.autograd.Function):
         _require(qkv, "qkv", (batch, seq_len, width))
         for t, name in ((cos, "cos"), (sin, "sin")):
             _require(t, name, (t.shape[0], dim), torch.float32)
-        wqf = None if wq is None else wq.detach().float().contiguous()
-        wkf = None if wk is None else wk.detach().float().contiguous()
+        wqf, wkf = (None if w is None else w if w.dtype is torch.float32 and w.is_contiguous()
+                    else w.detach().float().contiguous() for w in (wq, wk))
         q = torch.empty(batch, seq_len, heads, dim, dtype=DTYPE, device=qkv.device)
         k = torch.empty(batch, seq_len, kv_heads, dim, dtype=DTYPE, device=qkv.device)
         v = torch.empty_like(k)
@@ -661,7 +706,7 @@ class QKNormRope(torch.autograd.Function):
         grads = []
         for g, shp in zip((dq, dk, dv), shapes):
             g = torch.zeros(shp, dtype=DTYPE, device=qkv.device) if g is None else g
-            grads.append(g.to(DTYPE).contiguous())
+            grads.append(g if g.dtype is DTYPE and g.is_contiguous() else g.to(DTYPE).contiguous())
         dqkv = torch.empty_like(qkv)
         lib = _lib.load()
         norm = wqf is not None
@@ -720,8 +765,12 @@ class Attention(nn.Module):
         RoPE kernel; None when the projection is not bf16 (fp32 activations
         outside autocast keep the reference's fp32 norm and rotation)."""
         cfg = self.cfg
-        w = torch.cat((self.wq.weight, self.wk.weight, self.wv.weight), dim=0)
-        qkv = BF16Linear.apply(x, w) if _bf16_linear_applies(x) else F.linear(x, w)
+        ws = (self.wq.weight, self.wk.weight, self.wv.weight)
+        if _bf16_linear_applies(x) and all(_castable(w) and w.device == x.device for w in ws):
+            qkv = QKVLinear.apply(x, *ws)
+        else:
+            w = torch.cat(ws, dim=0)
+            qkv = BF16Linear.apply(x, w) if _bf16_linear_applies(x) else F.linear(x, w)
         if qkv.dtype != DTYPE or not qkv.is_cuda or cfg.head_dim != 128:
             return None
         qn = self.q_norm.weight if cfg.qk_norm else None
@@ -755,7 +804,8 @@ class Attention(nn.Module):
         fused = self.project_fused(x) if hip and x.is_cuda else None
         q, k, v = fused if fused is not None else self.project(x)
         if hip:
-            out = flash_attention(*(t.to(DTYPE).contiguous() for t in (q, k, v)), True, cfg.groups)
+            out = flash_attention(*(t if t.dtype is DTYPE and t.is_contiguous() else t.to(DTYPE).contiguous()
+                                    for t in (q, k, v)), True, cfg.groups)
             if not _skip_attn_out_cast():
                 out = out.to(x.dtype)
         else:

@@ -43,6 +43,7 @@ hipError_t launch_swiglu_gate_up(const void* x, const void* wg, const void* wu, 
 hipError_t launch_swiglu_grad(const void* dact, const void* gate, const void* up, void* dgate, void* dup,
                               int T, int F, long ld_out, hipStream_t stream);
 size_t lm_head_workspace_bytes(int T, int V);
+hipError_t launch_cast_bf16(const float* const src[4], const long n[4], void* dst, hipStream_t stream);
 hipError_t launch_lm_lse(const void* hidden, const void* weight, bool vocab_rows, const long long* targets,
                          long long ignore_index,
                          float* lse, float* tlogit_out, float* loss, void* workspace, int T, int d, int V,
@@ -692,6 +693,23 @@ int mm1_gemm(const void* x, int x_layout, long ldx, const void* w, int w_layout,
   if (need > 0 && (!workspace || workspace_bytes < need)) return MM1_E_WORKSPACE;
   mm1::GemmArgs a{x, ldx, x_layout, w, ldw, w_layout, w1, k_cut, out, out1, n_cut, ldo, out_f32 != 0, workspace, M, N, K};
   return from_hip(mm1::launch_gemm(a, static_cast<hipStream_t>(stream)));
+}
+
+int mm1_cast_bf16(const float* src0, long n0, const float* src1, long n1, const float* src2, long n2,
+                  const float* src3, long n3, void* dst, void* stream) {
+  const float* const src[4] = {src0, src1, src2, src3};
+  const long n[4] = {n0, n1, n2, n3};
+  if (!dst) return MM1_E_NULL;
+  long total = 0;
+  for (int j = 0; j < 4; ++j) {
+    if (n[j] < 0 || n[j] % 8 != 0 || n[j] > (1L << 40)) return MM1_E_SHAPE;
+    if (n[j] > 0 && !src[j]) return MM1_E_NULL;
+    if (n[j] > 0 && !aligned16(src[j])) return MM1_E_ALIGN;
+    total += n[j];
+  }
+  if (total == 0) return MM1_E_SHAPE;
+  if (!aligned16(dst)) return MM1_E_ALIGN;
+  return from_hip(mm1::launch_cast_bf16(src, n, dst, static_cast<hipStream_t>(stream)));
 }
 
 const char* mm1_attn_strerror(int code) {

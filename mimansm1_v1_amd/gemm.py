@@ -34,37 +34,42 @@ def applies(x, w) -> bool:
     both are k-major, N of 8, not x k-major with w k-contiguous) and was measured faster than
     hipBLASLt's GEMM at such a size (MI355X; T tokens, widths 1280 to 49152):
 
-    * with w k-major from M N K = 2.4e10 on: x k-major (weight gradients)
+    From M N K = 2.4e10 on:
+    * with w k-major: x k-major (weight gradients)
       1280 x 6656 x 16384 409 -> 309 us, 3328 x 1280 269 -> 174, 1280 x 49152
       1985 -> 1669, 1280 x 1280 130 -> 84; x k-contiguous 16384 x 1280 x 3328
-      161 -> 114 us, x 1792 91 -> 65.  Below (1792 x 1280 x 4096: 45 against
-      48 us) too few tiles or windows are left per CU.
+      161 -> 114 us, x 1792 91 -> 65;
     * both k-contiguous where 320-column tiles fill a round of the CUs
       (16384 x 1280 x 1280 63 -> 50 us, x 6656 225 -> 218, x 49152 1656 ->
       1558) or the reduction is long enough to split (1024 x 1280 x 49152
       331 -> 182 us); hipBLASLt is faster elsewhere (16384 x 3328 x 1280: 136
-      against 143 us)."""
+      against 143 us).
+    Below, too few tiles or windows are left per CU (1792 x 1280 x 4096, both
+    k-major: 45 against 48 us)."""
+    m, k = x.shape
+    n = w.shape[0]
+    if m * n * k < 24 * 10 ** 9:
+        return False
     lx, lw = _layout(x), _layout(w)
     if lx is None or lw is None or (lx[0] == COL and lw[0] == ROW):
         return False
-    m, k = x.shape
-    n = w.shape[0]
     if (k % 128 and lx[0] == ROW) or n % 8 or m < 1 or k < 1 or w.shape[1] != k or w.device != x.device:
         return False
     for (layout, ld), rows in ((lx, m), (lw, n)):
         if (256 * ld + k if layout == ROW else 64 * ld + rows) >= 1 << 30 or rows > 1 << 26:
             return False
     if lw[0] == COL:
-        return m * n * k >= 24 * 10 ** 9
+        return True
     return (n % 320 == 0 and m * n >= 230 * 256 * 320) or (k >= 16384 and m * n >= 16 * 256 * 256)
 
 
 def applies_joined(x, w, w1) -> bool:
     """applies() for product(x, w, w1): the joined width counts."""
-    if _layout(x) is None or _layout(w) is None or _layout(w) != _layout(w1) or w.shape != w1.shape:
-        return False
     k = w.shape[1]
-    return k % 64 == 0 and x.shape[1] == 2 * k and applies(x[:, :k], w) and (2 * k) % 128 == 0
+    if x.shape[0] * w.shape[0] * 2 * k < 24 * 10 ** 9:
+        return False
+    return (_layout(w) is not None and _layout(w) == _layout(w1) and w.shape == w1.shape
+            and k % 128 == 0 and x.shape[1] == 2 * k and applies(x[:, :k], w))
 
 
 def product(x, w, w1=None, out_dtype=DTYPE, split=None):
@@ -94,6 +99,6 @@ def product(x, w, w1=None, out_dtype=DTYPE, split=None):
     ptr = lambda t: None if t is None else t.data_ptr()
     rc = lib.mm1_gemm(x.data_ptr(), lx, ldx, w.data_ptr(), lw, ldw, ptr(w1), k_cut, out.data_ptr(), ptr(out1),
                       split or 0, out.stride(0), int(out_dtype == torch.float32), ptr(ws), ws_bytes, m, n, k,
-                      torch.cuda.current_stream(x.device).cuda_stream)
+                      torch._C._cuda_getCurrentRawStream(x.device.index))
     _lib.check(rc, "mm1_gemm")
     return out if split is None else (out, out1)
