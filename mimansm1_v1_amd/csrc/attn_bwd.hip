@@ -1229,6 +1229,215 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_dq_kernel(
   tail_reduce(red, tid, NW * 64);
 }
 
+// dQ of small grids: 8 waves as 8 / KS row waves x KS key groups, as the
+// key-split forward (attn_fwd_split_kernel): 128 keys per step, of which key
+// group kg takes 128 / KS; the groups' dQ are summed in group order through
+// LDS in fp32.  The arithmetic per key block is attn_dq_kernel's.
+// Whole backward with it, against the best of the other pairings (10 / 2 heads,
+// causal): 1 x 2048 122 -> 103 us (KS = 4), 2 x 2048 134 -> 126, 3 x 1365 107 ->
+// 101 (KS = 2), 1 x 512 56.0 -> 49.6; 8 x 2048 358 -> 385, where get_kernel's
+// search keeps the others.
+template <int KS, bool CAUSAL, bool F32OUT = false>
+__global__ __launch_bounds__(512, 1) void attn_dq_split_kernel(
+    const _Float16* __restrict__ q, const _Float16* __restrict__ k, const _Float16* __restrict__ v,
+    const _Float16* __restrict__ dO, const float* __restrict__ lse, const float* __restrict__ ndelta,
+    const float* __restrict__ scale, void* __restrict__ dq_out,
+    int B, int S, int H, int Hkv, int G, float scale2, float sm_scale, int n_tiles, TailReduce red,
+    const DispatchOrder ord) {
+  constexpr int RW = 8 / KS, BM = 32 * RW;
+  constexpr int BN = SPLIT_KEYS;
+  constexpr int NJ = BN / 32 / KS;          // 32-key blocks of a wave per step
+  constexpr int STAGE = 4 * TILE_BYTES;     // K tiles 0, 1; V tiles 0, 1
+  __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
+
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index (uniform)
+  const int rw = w % RW, kg = w / RW;
+  const int nbg = B * Hkv;
+  const int item = dispatch_item(ord);    // default order: blockIdx.x
+  if (item < 0) {                         // a launch slot without rows still sums its slice
+    tail_reduce(red, tid, 512);
+    return;
+  }
+  int tile = item / nbg;
+  if (CAUSAL) tile = n_tiles - 1 - tile;
+  const int bg = item % nbg;
+  const int b = bg / Hkv, g = bg % Hkv;
+  const int R = G * S;
+  const int r0 = tile * BM;
+  const int rw0 = r0 + 32 * rw;
+  const bool wave_active = rw0 < R;
+
+  const int last_row_wg = min(r0 + BM, R) - 1;
+  const int n_step = (CAUSAL ? min(S - 1, last_row_wg / G) : S - 1) / BN + 1;
+  const int pw_lo = rw0 / G;
+  const int pw_hi = CAUSAL ? min(S - 1, (min(rw0 + 32, R) - 1) / G) : S - 1;   // last key any row of the wave sees
+
+  const long kvstride = (long)Hkv * HD;
+  const _Float16* kbase = k + ((long)b * S * Hkv + g) * HD;
+  const _Float16* vbase = v + ((long)b * S * Hkv + g) * HD;
+  const uint32_t dma_off = tile_lane_off(kvstride, tid);
+  auto issue_step = [&](char* buf, int st) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int nk = st * BN + 64 * t;
+      if (nk < S) {                         // the second tile may lie past the sequence: never read then
+        tile_dma<8>(buf + t * TILE_BYTES, kbase + (long)nk * kvstride, kvstride, S - nk, dma_off, tid);
+        tile_dma<8>(buf + (2 + t) * TILE_BYTES, vbase + (long)nk * kvstride, kvstride, S - nk, dma_off, tid);
+      }
+    }
+  };
+  issue_step(smem, 0);
+
+  const int rr = rw0 + l32;
+  const int qp = rr / G;
+  const int hh = rr - qp * G;
+  const bool row_valid = rr < R;
+  const long roff = ((long)(b * S + qp) * H + g * G + hh) * HD;
+  f16x8 qreg[8], doreg[8];
+  float lse_i = INFINITY, dl_i = 0.f;
+  if (row_valid) {
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      qreg[ks] = *reinterpret_cast<const f16x8*>(q + roff + 16 * ks + 8 * h);
+      doreg[ks] = *reinterpret_cast<const f16x8*>(dO + roff + 16 * ks + 8 * h);
+    }
+    const long li = ((long)b * H + g * G + hh) * S + qp;
+    lse_i = lse[li];
+    dl_i = ndelta[li];   // -Delta
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) { pin(qreg[ks]); pin(doreg[ks]); }
+    __asm__ volatile("" : "+v"(lse_i), "+v"(dl_i));
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) { qreg[ks][t] = (_Float16)0.f; doreg[ks][t] = (_Float16)0.f; }
+    }
+  }
+  f32x16 negdl;   // the initial accumulator of every dP^T block: -Delta
+#pragma unroll
+  for (int r = 0; r < 16; ++r) negdl[r] = dl_i;
+  f32x16 dqacc[4];
+#pragma unroll
+  for (int db = 0; db < 4; ++db) dqacc[db] = zero16();
+  const LdsBases lb = make_lds_bases(lane);
+  wait_dma();
+  __syncthreads();
+
+  // the wave's keys of a step: blocks NJ kg .. of the four (tile NJ kg / 2)
+  const int kofs = NJ * kg * 32;
+  const int lofs = (kofs >> 6) * TILE_BYTES + ((kofs >> 5) & 1) * 8192;
+  auto step = [&](auto slot, int st) {
+    constexpr int P = decltype(slot)::value;
+    const char* kl = smem + P * STAGE + lofs;
+    const char* vl = kl + 2 * TILE_BYTES;
+    if (st + 1 < n_step) issue_step(smem + (P ^ 1) * STAGE, st + 1);
+    const int k0 = st * BN + kofs;
+    if (wave_active && k0 <= pw_hi) {
+      const bool need_mask = CAUSAL ? (k0 + 32 * NJ - 1 > pw_lo) : (k0 + 32 * NJ > S);
+#pragma unroll
+      for (int jb = 0; jb < NJ; ++jb) {
+        f32x16 sv = zero16(), dp = negdl;
+        constexpr int PF = MM1_DQ_PREFETCH;
+        f16x8 ka[PF + 1], va[PF + 1];
+#pragma unroll
+        for (int ks = 0; ks < PF; ++ks) {
+          ka[ks] = rows_a(kl, lb, jb, ks);
+          va[ks] = rows_a(vl, lb, jb, ks);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+          if (ks + PF < 8) {
+            ka[(ks + PF) % (PF + 1)] = rows_a(kl, lb, jb, ks + PF);
+            va[(ks + PF) % (PF + 1)] = rows_a(vl, lb, jb, ks + PF);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          sv = mfma32h(ka[ks % (PF + 1)], qreg[ks], sv);
+          dp = mfma32h(va[ks % (PF + 1)], doreg[ks], dp);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          float pr = exp2_fast(fmaf(sv[r], scale2, -lse_i));
+          if (need_mask) {
+            const int key = k0 + 32 * jb + 8 * (r >> 2) + 4 * h + (r & 3);
+            pr = (CAUSAL ? (key > qp) : (key >= S)) ? 0.f : pr;
+          }
+          sv[r] = pr * dp[r];
+        }
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh) {
+          const f16x8 sb = pack8(sv, 8 * kh);
+#pragma unroll
+          for (int db = 0; db < 4; ++db) dqacc[db] = mfma32h(tr_a(kl, lb, db, 2 * jb + kh), sb, dqacc[db]);
+        }
+      }
+    }
+    wait_dma();
+    lds_barrier();
+  };
+  for (int st = 0; st < n_step; st += 2) {
+    step(std::integral_constant<int, 0>{}, st);
+    if (st + 1 < n_step) step(std::integral_constant<int, 1>{}, st + 1);
+  }
+
+  // sum of the groups' dQ (the ring is free after the last barrier)
+  constexpr int MERGE = 16 * 1024;
+  static_assert((KS - 1) * RW * MERGE + RW * 8192 <= 2 * STAGE, "merge and staging fit the ring");
+  if (kg > 0) {
+    char* part = smem + ((kg - 1) * RW + rw) * MERGE;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+#pragma unroll
+      for (int a4 = 0; a4 < 4; ++a4) {
+        f32x4 x;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[c] = dqacc[db][4 * a4 + c];
+        *reinterpret_cast<f32x4*>(part + ((4 * db + a4) * 64 + lane) * 16) = x;
+      }
+    }
+  }
+  __syncthreads();
+  if (kg == 0 && wave_active) {
+#pragma unroll 1
+    for (int o = 1; o < KS; ++o) {
+      const char* src = smem + ((o - 1) * RW + rw) * MERGE;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+#pragma unroll
+        for (int a4 = 0; a4 < 4; ++a4) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(src + ((4 * db + a4) * 64 + lane) * 16);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) dqacc[db][4 * a4 + c] += x[c];
+        }
+      }
+    }
+    const float unscale = scale[0];   // 2^-E of do16
+    if constexpr (!F32OUT) {
+      store_tile_bf16(dqacc, unscale, smem + 2 * STAGE - (RW - rw) * 8192, lane, [&](int i) -> __bf16* {
+        const int r = rw0 + i;
+        if (r >= R) return nullptr;
+        const int p = r / G;
+        return static_cast<__bf16*>(dq_out) + ((long)(b * S + p) * H + g * G + (r - p * G)) * HD;
+      });
+    } else if (row_valid) {
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+#pragma unroll
+        for (int a4 = 0; a4 < 4; ++a4) {
+          f32x4 val;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) val[c] = dqacc[db][4 * a4 + c] * unscale;
+          *reinterpret_cast<f32x4*>(static_cast<float*>(dq_out) + roff + 32 * db + 8 * a4 + 4 * h) = val;
+        }
+      }
+    }
+  }
+  // dK/dV group sum slice (the partials were completed by an earlier launch)
+  tail_reduce(red, tid, 512);
+}
+
 // ---------------------------------------------------------------------------
 hipError_t launch_delta(const void* o, const void* dO, float* delta, int B, int S, int H,
                         hipStream_t stream) {
@@ -1415,9 +1624,25 @@ static void launch_dq_t(const BwdOperands& op, void* dq, int B, int S, int H, in
                        op.lse, op.ndelta, op.scale, dq, B, S, H, Hkv, G, scale2, sm_scale, n_qtiles, red, ord);
 }
 
+template <int KS, bool F32OUT>
+static void launch_dq_split(const BwdOperands& op, void* dq, int B, int S, int H, int Hkv, bool causal, float scale2,
+                            float sm_scale, TailReduce red, const DispatchOrder& ord, hipStream_t stream) {
+  const int G = H / Hkv, BM = 256 / KS;
+  const int n_qtiles = (G * S + BM - 1) / BM;
+  const int n_blocks = ord.n ? ord.n : n_qtiles * B * Hkv;
+  if (red.n_red > 0) red.n_red = min(red.n_red, n_blocks);
+  dim3 grid(n_blocks), block(512);
+  if (causal)
+    hipLaunchKernelGGL((attn_dq_split_kernel<KS, true, F32OUT>), grid, block, 0, stream, op.q, op.k, op.v, op.dO,
+                       op.lse, op.ndelta, op.scale, dq, B, S, H, Hkv, G, scale2, sm_scale, n_qtiles, red, ord);
+  else
+    hipLaunchKernelGGL((attn_dq_split_kernel<KS, false, F32OUT>), grid, block, 0, stream, op.q, op.k, op.v, op.dO,
+                       op.lse, op.ndelta, op.scale, dq, B, S, H, Hkv, G, scale2, sm_scale, n_qtiles, red, ord);
+}
+
 // dQ from the state and a prepared workspace.  variant: 0 = 4 waves x
 // 2-stage ring (two workgroups per CU), 1 = 8 waves x 3-stage ring (one per
-// CU).  reduce: also sum the dK/dV partials that tiling dkdv_variant left in
+// CU), 2, 3 = 8 waves over 128 / 64 rows, 2 / 4 key groups.  reduce: also sum the dK/dV partials that tiling dkdv_variant left in
 // the workspace into dk, dv (what launch_bwd_reduce does), in the dQ grid's
 // tail.  f32: dq (and dk, dv) are fp32.
 hipError_t launch_bwd_dq(const char* state, char* ws, void* dq, bool reduce, void* dk, void* dv, bool f32,
@@ -1429,7 +1654,13 @@ hipError_t launch_bwd_dq(const char* state, char* ws, void* dq, bool reduce, voi
   // with n_red = 1 << 30 every workgroup of the grid takes a slice
   const TailReduce red = make_reduce(partials, dk, dv, f32, B, S, H, Hkv, causal, dkdv_variant);
   const DispatchOrder& ord = dispatch_order(dq_grid(variant, B, S, H, Hkv), causal);
-  if (variant == 1) {
+  if (variant == 2) {
+    if (f32) launch_dq_split<2, true>(op, dq, B, S, H, Hkv, causal, scale2, sm_scale, red, ord, stream);
+    else launch_dq_split<2, false>(op, dq, B, S, H, Hkv, causal, scale2, sm_scale, red, ord, stream);
+  } else if (variant == 3) {
+    if (f32) launch_dq_split<4, true>(op, dq, B, S, H, Hkv, causal, scale2, sm_scale, red, ord, stream);
+    else launch_dq_split<4, false>(op, dq, B, S, H, Hkv, causal, scale2, sm_scale, red, ord, stream);
+  } else if (variant == 1) {
     if (f32) launch_dq_t<8, 3, true>(op, dq, B, S, H, Hkv, causal, scale2, sm_scale, red, ord, stream);
     else launch_dq_t<8, 3, false>(op, dq, B, S, H, Hkv, causal, scale2, sm_scale, red, ord, stream);
   } else {

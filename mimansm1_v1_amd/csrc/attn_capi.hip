@@ -79,6 +79,8 @@ const char* const kFwdTiles[] = {
     "block_M=256 block_N=64 waves=8 stages=2 schedule=pingpong",
     "block_M=128 block_N=64 waves=4 stages=2 schedule=ring",
     "block_M=256 block_N=64 waves=8 stages=3 schedule=ring",
+    "block_M=128 block_N=64 waves=8 stages=2 schedule=keysplit",
+    "block_M=64 block_N=64 waves=8 stages=2 schedule=keysplit",
 };
 const char* const kDkdvTiles[] = {
     "block_M=128 block_N=32 waves=8 stages=7 schedule=group",
@@ -87,6 +89,8 @@ const char* const kDkdvTiles[] = {
 const char* const kDqTiles[] = {
     "block_M=128 block_N=64 waves=4 stages=2 schedule=ring",
     "block_M=256 block_N=64 waves=8 stages=3 schedule=ring",
+    "block_M=128 block_N=64 waves=8 stages=2 schedule=keysplit",
+    "block_M=64 block_N=64 waves=8 stages=2 schedule=keysplit",
 };
 
 template <size_t N>

@@ -520,6 +520,204 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
   }
 }
 
+// Forward of small grids: 8 waves split as RW = 8 / KS row waves x KS key
+// groups over 32*RW packed rows, so that a shape with too few rows to fill
+// the CUs with 128-row workgroups has its key loop KS times shorter (what
+// bounds it there is the serial walk of the longest rows, not the matrix
+// cores).  Each step stages 128 keys (K and V, two 64-key tiles each, 2-slot
+// ring) of which key group kg takes 128 / KS; at the end the groups' (m, l, O)
+// are brought to the largest m of a row and summed in group order through
+// LDS, in fp32.  Forward with its K / V conversion, against the best of the
+// other tilings (10 / 2 heads, causal): 1 x 2048 51.8 -> 38.9 us (KS = 4),
+// 2 x 2048 55.5 -> 48.4, 3 x 1365 44.2 -> 39.4 (KS = 2), 1 x 512 22.5 -> 20.9;
+// where 128-row workgroups fill the CUs the merge and the single workgroup per
+// CU cost more than they save (8 x 2048: 113.6 against 136.7 us), so get_kernel's
+// search, not a rule, picks it per shape.
+template <int KS, bool CAUSAL, bool F32OUT = false>
+__global__ __launch_bounds__(512, 1) void attn_fwd_split_kernel(
+    const __bf16* __restrict__ q, const _Float16* __restrict__ k, const _Float16* __restrict__ v,
+    void* __restrict__ o_out, float* __restrict__ lse2, _Float16* __restrict__ q16, uint8_t* __restrict__ o_lo,
+    int B, int S, int H, int Hkv, int G, float scale2, int n_tiles, const DispatchOrder ord) {
+  constexpr int RW = 8 / KS, BM = 32 * RW;
+  constexpr int BN = SPLIT_KEYS;
+  constexpr int NJ = BN / 32 / KS;          // 32-key blocks of a wave per step
+  constexpr int STAGE = 4 * TILE_BYTES;     // K tiles 0, 1; V tiles 0, 1
+  __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
+
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index (uniform)
+  const int rw = w % RW, kg = w / RW;
+  const int nbg = B * Hkv;
+  const int item = dispatch_item(ord);     // default order: blockIdx.x
+  if (item < 0) return;
+  int tile = item / nbg;
+  if (CAUSAL) tile = n_tiles - 1 - tile;   // longest rows first
+  const int bg = item % nbg;
+  const int b = bg / Hkv, g = bg % Hkv;
+  const int R = G * S;
+  const int r0 = tile * BM;
+  const int rw0 = r0 + rw * 32;
+  const bool wave_active = rw0 < R;
+
+  const int last_row_wg = min(r0 + BM, R) - 1;
+  const int n_step = (CAUSAL ? min(S - 1, last_row_wg / G) : S - 1) / BN + 1;
+  const int pw_lo = rw0 / G;
+  const int pw_hi = CAUSAL ? min(S - 1, (min(rw0 + 32, R) - 1) / G) : S - 1;   // last key any row of the wave sees
+
+  const long kvstride = (long)Hkv * HD;
+  const _Float16* kbase = k + ((long)b * S * Hkv + g) * HD;
+  const _Float16* vbase = v + ((long)b * S * Hkv + g) * HD;
+  const uint32_t dma_off = tile_lane_off(kvstride, tid);
+  auto issue_step = [&](char* buf, int st) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int nk = st * BN + 64 * t;
+      if (nk < S) {                         // the second tile may lie past the sequence: never read then
+        tile_dma<8>(buf + t * TILE_BYTES, kbase + (long)nk * kvstride, kvstride, S - nk, dma_off, tid);
+        tile_dma<8>(buf + (2 + t) * TILE_BYTES, vbase + (long)nk * kvstride, kvstride, S - nk, dma_off, tid);
+      }
+    }
+  };
+  issue_step(smem, 0);
+
+  f16x8 qreg[8];
+  const int rr = rw0 + l32;
+  const int qpos = rr / G;
+  const int hq = rr - qpos * G;
+  const long qoff = ((long)(b * S + qpos) * H + g * G + hq) * HD;
+  _Float16* q16w = kg == 0 ? q16 : nullptr;
+  load_q16(qreg, q, q16w, qoff, rr < R, h);
+
+  f32x16 oacc[4];
+#pragma unroll
+  for (int db = 0; db < 4; ++db) oacc[db] = zero16();
+  float m_run = -INFINITY, l_run = 0.f;
+  const LdsBases lb = make_lds_bases(lane);
+  wait_dma();
+  __syncthreads();
+  store_q16(qreg, q16w, qoff, rr < R, h);
+
+  // the wave's keys of a step: blocks NJ kg .. of the four (tile NJ kg / 2)
+  const int kofs = NJ * kg * 32;
+  const int lofs = (kofs >> 6) * TILE_BYTES + ((kofs >> 5) & 1) * 8192;
+  auto step = [&](auto slot, int st) {
+    constexpr int P = decltype(slot)::value;
+    const char* kl = smem + P * STAGE + lofs;
+    const char* vl = kl + 2 * TILE_BYTES;
+    if (st + 1 < n_step) issue_step(smem + (P ^ 1) * STAGE, st + 1);
+    const int k0 = st * BN + kofs;
+    if (wave_active && k0 <= pw_hi) {
+      f32x16 sacc[NJ];
+#pragma unroll
+      for (int jb = 0; jb < NJ; ++jb) sacc[jb] = zero16();
+      if constexpr (NJ == 2) {
+        rows_chain2(kl, lb, qreg, sacc);
+      } else {
+        mfma_chain<8, 2>([&](int ks) MM1_INLINE { return rows_a(kl, lb, 0, ks); },
+                         [&](int ks, const f16x8& a) MM1_INLINE { sacc[0] = mfma32h(a, qreg[ks], sacc[0]); },
+                         [](int) MM1_INLINE {});
+      }
+      if (CAUSAL ? (k0 + 32 * NJ - 1 > pw_lo) : (k0 + 32 * NJ > S)) {
+#pragma unroll
+        for (int jb = 0; jb < NJ; ++jb) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = k0 + 32 * jb + 8 * (r >> 2) + 4 * h + (r & 3);
+            sacc[jb][r] = (CAUSAL ? (key > qpos) : (key >= S)) ? -INFINITY : sacc[jb][r];
+          }
+        }
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int jb = 0; jb < NJ; ++jb) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sacc[jb][r]);
+      }
+      mx = xhalf_max(mx);
+      const float m_new = fmaxf(m_run, mx);
+      // (m_new == m_run covers rows that have seen no key yet: both -inf)
+      if (__any(m_new != m_run && !((m_new - m_run) * scale2 <= kRescaleThreshold))) {
+        const float alpha = (m_run == m_new) ? 1.f : exp2_fast((m_run - m_new) * scale2);
+        l_run *= alpha;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
+        m_run = m_new;
+      }
+      const float ms = (m_run == -INFINITY) ? 0.f : m_run * scale2;
+      float sum = 0.f;
+#pragma unroll
+      for (int jb = 0; jb < NJ; ++jb) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float pr = exp2_fast(fmaf(sacc[jb][r], scale2, -ms));
+          sacc[jb][r] = pr;
+          sum += pr;
+        }
+      }
+      l_run += sum;
+#pragma unroll
+      for (int ks = 0; ks < 2 * NJ; ++ks) {
+        const f16x8 pb = pack8(sacc[ks >> 1], 8 * (ks & 1));
+#pragma unroll
+        for (int db = 0; db < 4; ++db) oacc[db] = mfma32h(tr_a(vl, lb, db, ks), pb, oacc[db]);
+      }
+    }
+    wait_dma();
+    lds_barrier();
+  };
+  for (int st = 0; st < n_step; st += 2) {
+    step(std::integral_constant<int, 0>{}, st);
+    if (st + 1 < n_step) step(std::integral_constant<int, 1>{}, st + 1);
+  }
+
+  // Merge (the ring is free after the last barrier): m of every wave, then O
+  // and l of the groups after the first, 16.25 KiB per wave.
+  constexpr int MERGE = 16 * 1024 + 256;
+  float* ms = reinterpret_cast<float*>(smem);
+  ms[w * 64 + lane] = m_run;
+  __syncthreads();
+  float m_all = m_run;
+#pragma unroll
+  for (int o = 0; o < KS; ++o) m_all = fmaxf(m_all, ms[(o * RW + rw) * 64 + lane]);
+  const float alpha = m_run == m_all ? 1.f : exp2_fast((m_run - m_all) * scale2);   // m_run = -inf: 0
+  l_run *= alpha;
+#pragma unroll
+  for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
+  char* part = smem + 2048 + ((kg - 1) * RW + rw) * MERGE;
+  if (kg > 0) {
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+#pragma unroll
+      for (int a4 = 0; a4 < 4; ++a4) {
+        f32x4 x;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[c] = oacc[db][4 * a4 + c];
+        *reinterpret_cast<f32x4*>(part + ((4 * db + a4) * 64 + lane) * 16) = x;
+      }
+    }
+    *reinterpret_cast<float*>(part + 16 * 1024 + lane * 4) = l_run;
+  }
+  __syncthreads();
+  if (kg > 0 || !wave_active) return;
+#pragma unroll 1
+  for (int o = 1; o < KS; ++o) {
+    const char* src = smem + 2048 + ((o - 1) * RW + rw) * MERGE;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+#pragma unroll
+      for (int a4 = 0; a4 < 4; ++a4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(src + ((4 * db + a4) * 64 + lane) * 16);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) oacc[db][4 * a4 + c] += x[c];
+      }
+    }
+    l_run += *reinterpret_cast<const float*>(src + 16 * 1024 + lane * 4);
+  }
+  static_assert(2048 + (KS - 1) * RW * MERGE + RW * 8192 <= 2 * STAGE, "merge and staging fit the ring");
+  store_fwd_rows<F32OUT>(oacc, m_all, l_run, scale2, o_out, o_lo, lse2, smem + 2 * STAGE - (RW - rw) * 8192, lane, b,
+                         g, S, H, G, R, rw0);
+}
+
 // K, V -> k16, v16 (with max|V| partials in vmax when it is not null).
 hipError_t launch_cvt_kv(const void* k, const void* v, _Float16* k16, _Float16* v16, float* kmax, float* vmax,
                          long n, hipStream_t stream) {
@@ -561,6 +759,21 @@ static void launch_fwd_t(const __bf16* q, const _Float16* k, const _Float16* v, 
                        q16, o_lo, B, S, H, Hkv, G, scale2, n_tiles, ord);
 }
 
+template <int KS, bool F32OUT>
+static void launch_fwd_split(const __bf16* q, const _Float16* k, const _Float16* v, void* o, float* lse2,
+                             _Float16* q16, uint8_t* o_lo, int B, int S, int H, int Hkv, bool causal, float scale2,
+                             const DispatchOrder& ord, hipStream_t stream) {
+  const int G = H / Hkv, BM = 256 / KS;
+  const int n_tiles = (G * S + BM - 1) / BM;
+  dim3 grid(ord.n ? ord.n : n_tiles * B * Hkv), block(512);
+  if (causal)
+    hipLaunchKernelGGL((attn_fwd_split_kernel<KS, true, F32OUT>), grid, block, 0, stream, q, k, v, o, lse2, q16,
+                       o_lo, B, S, H, Hkv, G, scale2, n_tiles, ord);
+  else
+    hipLaunchKernelGGL((attn_fwd_split_kernel<KS, false, F32OUT>), grid, block, 0, stream, q, k, v, o, lse2, q16,
+                       o_lo, B, S, H, Hkv, G, scale2, n_tiles, ord);
+}
+
 template <bool F32OUT>
 static void launch_fwd_v(const __bf16* qp, const _Float16* kp, const _Float16* vp, void* o, float* lse2,
                          _Float16* q16, uint8_t* o_lo, int B, int S, int H, int Hkv, bool causal, float scale2,
@@ -576,6 +789,10 @@ static void launch_fwd_v(const __bf16* qp, const _Float16* kp, const _Float16* v
     else
       hipLaunchKernelGGL((attn_fwd_pp_kernel<false, F32OUT>), grid, block, 0, stream, qp, kp, vp, o, lse2, q16,
                          o_lo, B, S, H, Hkv, G, scale2, n_tiles, ord);
+  } else if (variant == 3) {
+    launch_fwd_split<2, F32OUT>(qp, kp, vp, o, lse2, q16, o_lo, B, S, H, Hkv, causal, scale2, ord, stream);
+  } else if (variant == 4) {
+    launch_fwd_split<4, F32OUT>(qp, kp, vp, o, lse2, q16, o_lo, B, S, H, Hkv, causal, scale2, ord, stream);
   } else if (variant == 2) {
     launch_fwd_t<8, 3, F32OUT>(qp, kp, vp, o, lse2, q16, o_lo, B, S, H, Hkv, causal, scale2, ord, stream);
   } else {
@@ -588,7 +805,8 @@ static void launch_fwd_v(const __bf16* qp, const _Float16* kp, const _Float16* v
 // and o_lo for the backward.  F32 (o is float*): fp32 O, same kernels.
 // variant: 0 = attn_fwd_pp_kernel (8 waves, two groups half a tile apart),
 //          1 = 4 waves x 2-stage ring (two workgroups per CU),
-//          2 = 8 waves x 3-stage ring (one workgroup per CU).
+//          2 = 8 waves x 3-stage ring (one workgroup per CU),
+//          3, 4 = 8 waves over 128 / 64 rows, 2 / 4 key groups.
 hipError_t launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse2, bool f32,
                       _Float16* q16, _Float16* k16, _Float16* v16, uint8_t* o_lo, float* vmax, bool save,
                       int B, int S, int H, int Hkv, bool causal, float sm_scale, int variant, hipStream_t stream) {

@@ -58,8 +58,8 @@ struct GridShape {
 };
 
 // The grid of the forward launcher for a tiling index (1 = 128 rows, 2
-// workgroups per CU; 0, 2 = 256 rows, 1 per CU) and of the dQ launcher
-// (0 = 128 rows, 2 per CU; 1 = 256 rows, 1 per CU).
+// workgroups per CU; 0, 2 = 256 rows, 3 = 128, 4 = 64, 1 per CU) and of the
+// dQ launcher (0 = 128 rows, 2 per CU; 1 = 256 rows, 2 = 128, 3 = 64, 1 per CU).
 GridShape row_block_grid(int variant, int B, int S, int H, int Hkv);
 GridShape dq_grid(int variant, int B, int S, int H, int Hkv);
 

@@ -293,11 +293,13 @@ const DispatchOrder& default_order() {
 }  // namespace
 
 GridShape row_block_grid(int variant, int B, int S, int H, int Hkv) {
-  return {B, S, H, Hkv, variant == 1 ? 128 : 256, variant == 1 ? 2 : 1};
+  const int rows = variant == 4 ? 64 : variant == 1 || variant == 3 ? 128 : 256;
+  return {B, S, H, Hkv, rows, variant == 1 ? 2 : 1};
 }
 
 GridShape dq_grid(int variant, int B, int S, int H, int Hkv) {
-  return {B, S, H, Hkv, variant == 0 ? 128 : 256, variant == 0 ? 2 : 1};
+  const int rows = variant == 3 ? 64 : variant == 0 || variant == 2 ? 128 : 256;
+  return {B, S, H, Hkv, rows, variant == 0 ? 2 : 1};
 }
 
 const DispatchOrder& dispatch_order_for(const GridShape& g, bool causal, int cus) {

@@ -67,6 +67,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr int HD = 128;            // head_dim supported by the kernels
 constexpr int TILE_ROWS = 64;      // rows in one LDS tile
 constexpr int TILE_BYTES = TILE_ROWS * HD * 2;   // 16 KiB
+constexpr int SPLIT_KEYS = 128;    // keys per step of the key-split kernels
 
 __device__ __forceinline__ f32x16 mfma32(const bf16x8& a, const bf16x8& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
