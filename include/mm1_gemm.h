@@ -24,9 +24,14 @@ extern "C" {
 #define MM1_GEMM_ROW 0
 #define MM1_GEMM_COL 1
 
-/* Bytes of scratch mm1_gemm needs for this shape (0 for most): fp32 partial
- * sums where a few leftover tiles are split along K over all CUs. */
-size_t mm1_gemm_workspace_size(int M, int N, int K);
+/* Bytes of scratch mm1_gemm needs for this shape, with (joined) or without a
+ * w1 (0 for many): fp32 partial
+ * sums where K is split over several workgroups. */
+size_t mm1_gemm_workspace_size(int M, int N, int K, int joined);
+
+/* Modelled time of mm1_gemm at this shape on the current device, in us
+ * (negative for sizes it refuses). */
+double mm1_gemm_estimate_us(int M, int N, int K);
 
 /* out[m][n] = sum_k x(m, k) w(n, k): bf16 operands, fp32 accumulation over
  * all of K, rounded once to bf16 (out_f32 = 0) or stored in fp32 (1).

@@ -61,7 +61,8 @@ SIGNATURES = {
                                       _c_int, _c_int, _c_int, _vp]),
     "mm1_lm_head_dlogits_rows": (_c_int, [_vp, _vp, _vp, ctypes.c_longlong, _vp, _vp, _vp, ctypes.c_long,
                                           _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
-    "mm1_gemm_workspace_size": (_c_size, [_c_int, _c_int, _c_int]),
+    "mm1_gemm_workspace_size": (_c_size, [_c_int] * 4),
+    "mm1_gemm_estimate_us": (ctypes.c_double, [_c_int, _c_int, _c_int]),
     "mm1_gemm": (_c_int, [_vp, _c_int, ctypes.c_long, _vp, _c_int, ctypes.c_long, _vp, _c_int, _vp, _vp, _c_int,
                           ctypes.c_long, _c_int, _vp, _c_size, _c_int, _c_int, _c_int, _vp]),
     "mm1_cast_bf16": (_c_int, [_vp, ctypes.c_long] * 4 + [_vp, _vp]),

@@ -669,10 +669,16 @@ int mm1_lm_head_dlogits_rows(const void* hidden, const void* weight, const long 
                          v0, vn, stream);
 }
 
-size_t mm1_gemm_workspace_size(int M, int N, int K) {
-  if (M < 1 || N < 1 || K < 1 || K > (1 << 28)) return 0;
-  return mm1::gemm_workspace_bytes(M, N, K);
+static bool gemm_sizes_ok(int M, int N, int K) {
+  return M >= 1 && N >= 1 && K >= 1 && M <= (1 << 28) && N <= (1 << 28) && K <= (1 << 28) &&
+         ((long)M + 255) / 256 * (((long)N + 255) / 256) <= (1L << 24);
 }
+
+size_t mm1_gemm_workspace_size(int M, int N, int K, int joined) {
+  return gemm_sizes_ok(M, N, K) ? mm1::gemm_workspace_bytes(M, N, K, joined != 0) : 0;
+}
+
+double mm1_gemm_estimate_us(int M, int N, int K) { return gemm_sizes_ok(M, N, K) ? mm1::gemm_estimate_us(M, N, K) : -1.; }
 
 int mm1_gemm(const void* x, int x_layout, long ldx, const void* w, int w_layout, long ldw, const void* w1,
              int k_cut, void* out, void* out1, int n_cut, long ldo, int out_f32, void* workspace,
@@ -680,8 +686,7 @@ int mm1_gemm(const void* x, int x_layout, long ldx, const void* w, int w_layout,
   if (!x || !w || !out) return MM1_E_NULL;
   const bool xc = x_layout == MM1_GEMM_COL, wc = w_layout == MM1_GEMM_COL;
   if ((x_layout != MM1_GEMM_ROW && !xc) || (w_layout != MM1_GEMM_ROW && !wc) || (xc && !wc)) return MM1_E_SHAPE;
-  if (M < 1 || N < 1 || K < 1 || K > (1 << 28) || (!xc && K % 128 != 0) || N % 8 != 0 || (xc && M % 8 != 0))
-    return MM1_E_SHAPE;
+  if (!gemm_sizes_ok(M, N, K) || (!xc && K % 128 != 0) || N % 8 != 0 || (xc && M % 8 != 0)) return MM1_E_SHAPE;
   if (w1 ? k_cut < 64 || k_cut % 64 != 0 || k_cut >= K : k_cut != 0) return MM1_E_SHAPE;
   if (out1 ? n_cut < 64 || n_cut % 64 != 0 || n_cut >= N : n_cut != 0) return MM1_E_SHAPE;
   const int w_k = w1 ? (k_cut > K - k_cut ? k_cut : K - k_cut) : K;             // longest k run in one matrix
@@ -689,11 +694,10 @@ int mm1_gemm(const void* x, int x_layout, long ldx, const void* w, int w_layout,
   if (ldx < (xc ? M : K) || ldw < (wc ? N : w_k) || ldo < out_n || ldx % 8 || ldw % 8 || ldo % 8) return MM1_E_SHAPE;
   if (!mm1::gemm_operand_fits(x_layout, ldx, M, K) || !mm1::gemm_operand_fits(w_layout, ldw, N, w_k))
     return MM1_E_SHAPE;
-  if (M > (1 << 28) || N > (1 << 28) || ((long)M + 255) / 256 * (((long)N + 255) / 256) > (1L << 24)) return MM1_E_SHAPE;
   if (!aligned16(x) || !aligned16(w) || (w1 && !aligned16(w1)) || !aligned16(out) || (out1 && !aligned16(out1)) ||
       (workspace && !aligned16(workspace)))
     return MM1_E_ALIGN;
-  const size_t need = mm1::gemm_workspace_bytes(M, N, K);
+  const size_t need = mm1::gemm_workspace_bytes(M, N, K, w1 != nullptr);
   if (need > 0 && (!workspace || workspace_bytes < need)) return MM1_E_WORKSPACE;
   mm1::GemmArgs a{x, ldx, x_layout, w, ldw, w_layout, w1, k_cut, out, out1, n_cut, ldo, out_f32 != 0, workspace, M, N, K};
   return from_hip(mm1::launch_gemm(a, static_cast<hipStream_t>(stream)));

@@ -72,6 +72,30 @@ __device__ __forceinline__ void store_rows32(const Output& o, char* lds, int lan
   }
 }
 
+// One 32 x 32 block from val(q), the f32x4 of columns 8q + 4(lane/32) .. +3 of
+// row lane & 31.
+template <bool F32, class Val>
+__device__ __forceinline__ void store_block32(const Output& o, char* lds, int lane, long row0, int col0, Val&& val) {
+  if constexpr (F32) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float* p = out_at<float>(o, row0 + (lane & 31), col0 + 8 * q + 4 * (lane >> 5));
+      if (p) *reinterpret_cast<f32x4*>(p) = val(q);
+    }
+  } else {
+    gemm::store_block64<false>(
+        lds, lane,
+        [&](int q) {
+          const f32x4 x = val(q);
+          bf16x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = (__bf16)x[e];
+          return v;
+        },
+        [&](int r) { return out_at<__bf16>(o, row0 + r, col0); }, [&](int c) { return col0 + 8 * c < o.N; });
+  }
+}
+
 __device__ __forceinline__ f32x4 quad(const f32x16& a, int q) {
   f32x4 v;
 #pragma unroll
@@ -151,14 +175,67 @@ __global__ __launch_bounds__(64 * S::TI) void split_sum_kernel(const float* __re
                               nb * S::BN + 32 * S::TJ * wn, [&](int b, int q) { return sum[b][q]; });
 }
 
+// Small tiles (gemm_core.h): workgroup item = split * tiles + tile, an XCD's
+// workgroups on consecutive items; with several splits of k each writes its
+// fp32 partial tile ([wave][q][lane] x 4 floats) to slot tile * splits + split
+// and small_sum_kernel adds them in split order.  Bound by the latency of one
+// tile's k walk (0.35 us a window): 77 x 3328 x 1280 12.1 us a call, 300 x 1280 x
+// 1280 11.3, 77 x 1280 x 6656 (15 splits) 15.5, where torch's GEMM takes 21 us
+// (its host work).
+template <gemm::Layout LX, gemm::Layout LW, bool F32>
+__global__ __launch_bounds__(256) void gemm_small_kernel(const gemm::Problem p, const Output o, float* part,
+                                                         int splits) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int tiles = p.n_mblk * p.n_nblk, total = tiles * splits, per = (total + 7) / 8;
+  const int j = (int)(blockIdx.x >> 3), item = (int)(blockIdx.x & 7) * per + j;
+  if (j >= per || item >= total) return;
+  const int split = item / tiles, t = item - split * tiles;
+  const int nb = t / p.n_mblk, mb = t - nb * p.n_mblk;
+  const int n_win = (p.K + gemm::BK - 1) / gemm::BK;
+  const int w0 = (int)((long)split * n_win / splits), w1 = (int)((long)(split + 1) * n_win / splits);
+  f32x16 acc[1];
+  gemm::run_small<LX, LW, false>(p, smem, mb, nb, w0, w1 - w0, acc);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (splits > 1) {
+    float* dst = part + ((((long)t * splits + split) * 4 + w) * 4 * 64 + lane) * 4;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) *reinterpret_cast<f32x4*>(dst + q * 256) = quad(acc[0], q);
+    return;
+  }
+  store_block32<F32>(o, smem + 2048 * w, lane, (long)mb * gemm::SMALL + 32 * (w & 1), nb * gemm::SMALL + 32 * (w >> 1),
+                     [&](int q) { return quad(acc[0], q); });
+}
+
+template <bool F32>
+__global__ __launch_bounds__(256) void small_sum_kernel(const float* __restrict__ part, const Output o, int n_mblk,
+                                                        int splits) {
+  __shared__ __attribute__((aligned(1024))) char smem[4 * 2048];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t = blockIdx.x, nb = t / n_mblk, mb = t - nb * n_mblk;
+  f32x4 sum[4] = {};
+  for (int s = 0; s < splits; ++s) {
+    const float* src = part + ((((long)t * splits + s) * 4 + w) * 4 * 64 + lane) * 4;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sum[q] += *reinterpret_cast<const f32x4*>(src + q * 256);
+  }
+  store_block32<F32>(o, smem + 2048 * w, lane, (long)mb * gemm::SMALL + 32 * (w & 1), nb * gemm::SMALL + 32 * (w >> 1),
+                     [&](int q) { return sum[q]; });
+}
+
 namespace {
 
 // Cost of a plan in windows of a 256-column tile (~1.4 us each).
 constexpr double SPLIT_COST = 28;   // writing the partial sums and adding them: ~40 us, measured at 65 to 320 tiles
+constexpr double FILL_COST = 7;     // launch, first window and epilogue, 10 us
 constexpr double HALF_COST = 0.85;  // a half tile (WholeTiles): its copies are a whole tile's
+
+// Small tiles, in us: the launch and the ring's first fill, each round of
+// workgroups, each of its windows, and the sum of the splits.
+constexpr double SMALL_FILL = 3, SMALL_ROUND = 1.5, SMALL_WINDOW = 0.35, SMALL_SUM = 4, WINDOW_US = 1.4;
 
 struct Plan {
   bool wide320;
+  int splits;                       // small tiles: splits of k (0: large tiles)
   int n_mblk, n_nblk, grid, left;   // left: tiles split along k (0: none)
   double cost;
   size_t part_bytes;
@@ -173,9 +250,9 @@ Plan plan_of(int bn, int M, int N, int K, int n_g) {
   const int left = (int)(total % n_g);
   const double tile = (double)gemm::windows_of(K) * bn / 256, full = (double)(total / n_g);
   const double last = left == 0 ? 0 : 2 * left <= n_g ? HALF_COST : 1;
-  p.cost = (full + last) * tile;
+  p.cost = FILL_COST + (full + last) * tile;
   p.grid = gemm::persistent_grid(n_g, (int)total);
-  const double split = (full + (double)left / n_g) * tile + SPLIT_COST;
+  const double split = FILL_COST + (full + (double)left / n_g) * tile + SPLIT_COST;
   if (left > 0 && split < p.cost) {
     p.cost = split;
     p.left = left;
@@ -185,11 +262,37 @@ Plan plan_of(int bn, int M, int N, int K, int n_g) {
   return p;
 }
 
-// The tile width and the split of the leftover tiles, by modelled cost.
-Plan make_plan(int M, int N, int K, int cus) {
+Plan small_plan(int M, int N, int K, int n_g) {
+  Plan p{};
+  p.n_mblk = (M + gemm::SMALL - 1) / gemm::SMALL;
+  p.n_nblk = (N + gemm::SMALL - 1) / gemm::SMALL;
+  const long tiles = (long)p.n_mblk * p.n_nblk;
+  const int n_win = (K + gemm::BK - 1) / gemm::BK;
+  auto us = [&](int splits) {
+    const double rounds = (double)((tiles * splits + n_g - 1) / n_g);
+    return SMALL_FILL + rounds * (SMALL_ROUND + SMALL_WINDOW * ((n_win + splits - 1) / splits)) +
+           (splits > 1 ? SMALL_SUM : 0);
+  };
+  p.splits = 1;
+  double best = us(1);
+  for (int s = 2; s <= 16 && s * 4 <= n_win && s * tiles <= 2 * n_g; ++s) {
+    if (us(s) < best) {
+      best = us(s);
+      p.splits = s;
+    }
+  }
+  p.cost = best / WINDOW_US;
+  p.grid = (int)((tiles * p.splits + 7) / 8 * 8);
+  p.part_bytes = p.splits > 1 ? (size_t)tiles * p.splits * gemm::SMALL * gemm::SMALL * 4 : 0;
+  return p;
+}
+
+// The tile size, and the split of the leftover tiles or of k, by modelled cost.
+Plan make_plan(int M, int N, int K, int cus, bool joined) {
   const int n_g = ((cus > 0 ? cus : 256) + 7) & ~7;
-  const Plan a = plan_of(256, M, N, K, n_g), b = plan_of(320, M, N, K, n_g);
-  return b.cost < a.cost ? b : a;
+  const Plan a = plan_of(256, M, N, K, n_g), b = plan_of(320, M, N, K, n_g), c = small_plan(M, N, K, n_g);
+  const Plan& large = b.cost < a.cost ? b : a;
+  return c.cost < large.cost && !joined ? c : large;      // the small tiles take one W only
 }
 
 hipError_t cu_count(int& cus) {
@@ -237,6 +340,28 @@ hipError_t launch_s(const Launch& l) {
   return hipGetLastError();
 }
 
+template <gemm::Layout LX, gemm::Layout LW, bool F32>
+hipError_t launch_small_t(const Launch& l) {
+  auto kern = gemm_small_kernel<LX, LW, F32>;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, gemm::SMALL_LDS);
+  if (e != hipSuccess) return e;
+  auto part = static_cast<float*>(l.a.workspace);
+  hipLaunchKernelGGL(kern, dim3(l.plan.grid), dim3(256), gemm::SMALL_LDS, l.stream, l.p, l.o, part, l.plan.splits);
+  if (l.plan.splits > 1)
+    hipLaunchKernelGGL((small_sum_kernel<F32>), dim3(l.plan.n_mblk * l.plan.n_nblk), dim3(256), 0, l.stream,
+                       static_cast<const float*>(part), l.o, l.plan.n_mblk, l.plan.splits);
+  return hipGetLastError();
+}
+
+template <bool F32>
+hipError_t launch_small(const Launch& l) {
+  if (l.a.x_layout == gemm::ROW)
+    return l.a.w_layout == gemm::ROW ? launch_small_t<gemm::ROW, gemm::ROW, F32>(l)
+                                     : launch_small_t<gemm::ROW, gemm::COL, F32>(l);
+  return launch_small_t<gemm::COL, gemm::COL, F32>(l);
+}
+
 template <class S>
 hipError_t launch_o(const Launch& l) {
   if (l.a.f32) return launch_s<S, true, false>(l);
@@ -249,21 +374,28 @@ bool gemm_operand_fits(int layout, long ld, int n, int K) {
   return gemm::offsets_fit(static_cast<gemm::Layout>(layout), ld, n, K);
 }
 
-size_t gemm_workspace_bytes(int M, int N, int K) {
+size_t gemm_workspace_bytes(int M, int N, int K, bool joined) {
   int cus = 0;
   if (cu_count(cus) != hipSuccess) cus = 256;
-  return make_plan(M, N, K, cus).part_bytes;
+  return make_plan(M, N, K, cus, joined).part_bytes;
+}
+
+double gemm_estimate_us(int M, int N, int K) {
+  int cus = 0;
+  if (cu_count(cus) != hipSuccess) cus = 256;
+  return make_plan(M, N, K, cus, false).cost * WINDOW_US;
 }
 
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t stream) {
   int cus = 0;
   hipError_t e = cu_count(cus);
   if (e != hipSuccess) return e;
-  const Plan plan = make_plan(a.M, a.N, a.K, cus);
+  const Plan plan = make_plan(a.M, a.N, a.K, cus, a.w1 != nullptr);
   const gemm::Problem p{{static_cast<const __bf16*>(a.x), a.ldx, a.M}, {static_cast<const __bf16*>(a.w), a.ldw, a.N},
                         static_cast<const __bf16*>(a.w1), a.k_cut, a.K, plan.n_mblk, plan.n_nblk};
   const Output o{a.out, a.out1, a.ldo, a.M, a.N, a.out1 ? a.n_cut : a.N};
   const Launch l{a, plan, p, o, stream};
+  if (plan.splits > 0) return a.f32 ? launch_small<true>(l) : launch_small<false>(l);
   return plan.wide320 ? launch_o<gemm::Wide320>(l) : launch_o<gemm::Wide256>(l);
 }
 

@@ -580,5 +580,166 @@ __device__ __forceinline__ void store_rows128(char* lds, int lane, Val&& val, Ro
         lds, lane, [&](int b, int q) { return val(i, b, q); }, [&](int r) { return row(32 * i + r); }, chunk_ok);
 }
 
+// ---------------------------------------------------------------------------
+// Small tiles: 64 rows x 64 columns per workgroup of 4 waves, for products
+// with too few 256-wide tiles to occupy the CUs, whose time is the latency of
+// one workgroup's walk over k.  An eight-slot ring (16 KiB per 64-k window)
+// keeps seven windows in flight, against one in the large tile; the LDS panels
+// and swizzles are the same.  Wave w of the plain form owns the 32 x 32 block
+// (w & 1, w >> 1); PAIRED (32 columns of each of two matrices) gives wave w
+// rows 32 (w & 1) and both column blocks for the k steps 2 (w >> 1), +1 of
+// every window, so that a lane holds the same (row, column) of both; the two k
+// halves are summed through LDS (small_sum_halves).
+constexpr int SMALL = 64, SMALL_WAVES = 4, SMALL_SLOTS = 8;
+constexpr int SMALL_SLOT = 4 * PANEL;                     // X panels 0, 1; W panels 0, 1
+constexpr int SMALL_LDS = SMALL_SLOTS * SMALL_SLOT;
+
+// Fragment reads of one 32-row (column) block with a run-time slot offset.
+template <Layout L>
+struct SmallFrag;
+
+template <>
+struct SmallFrag<ROW> {
+  uint32_t base;
+  __device__ __forceinline__ SmallFrag(int lane, uint32_t region, int blk) {
+    const int l32 = lane & 31, h = lane >> 5;
+    base = region + blk * PANEL + l32 * 128 + 16 * (h ^ ((l32 >> 1) & 7));
+  }
+  __device__ __forceinline__ bf16x8 get(int slot_off, int kk) const {
+    return *reinterpret_cast<const MM1_LDS bf16x8*>((const MM1_LDS char*)(uintptr_t)((base ^ (32 * kk)) + slot_off));
+  }
+};
+
+template <>
+struct SmallFrag<COL> {
+  uint32_t off[2];
+  __device__ __forceinline__ SmallFrag(int lane, uint32_t region, int blk) {
+    const int h = lane >> 5, g = (lane >> 4) & 1, j = lane & 15, jj = j >> 2;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int row = 8 * h + 4 * r + jj, s = (((jj >> 1) & 1) << 2) | ((2 * h + r) & 3);
+      off[r] = region + row * 128 + 16 * ((4 * blk + 2 * g + ((j & 3) >> 1)) ^ s) + 8 * (j & 1);
+    }
+  }
+  __device__ __forceinline__ bf16x8 get(int slot_off, int kk) const {
+    bf16x8 out;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const bf16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+          (MM1_LDS bf16x4*)((const MM1_LDS char*)(uintptr_t)off[r] + (slot_off + (kk >> 1) * PANEL + 2048 * (kk & 1))));
+#pragma unroll
+      for (int q = 0; q < 4; ++q) out[4 * r + q] = v[q];
+    }
+    return out;
+  }
+};
+
+// Windows w0 .. w0 + nw - 1 of the tile (mb, nb): acc[0] the wave's block, or
+// (PAIRED) acc[0], acc[1] the blocks of the two matrices over the wave's k
+// half.  All 256 threads call it; it ends with a barrier, so the ring is free.
+template <Layout LX, Layout LW, bool PAIRED>
+__device__ __forceinline__ void run_small(const Problem& p, char* smem, int mb, int nb, int w0, int nw,
+                                          f32x16 (&acc)[PAIRED ? 2 : 1]) {
+  constexpr bool RAGGED_K = LX == COL && LW == COL;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(smem));
+  // copies: piece w (8 LDS rows) of X panels 0, 1 and W panels 0, 1
+  const int lr = 8 * w + (lane >> 3);
+  const int crow = 8 * ((lane & 7) ^ ((lr >> 1) & 7));
+  const int ccol = 8 * ((lane & 7) ^ ((((lr >> 1) & 1) << 2) | ((lr >> 2) & 3)));
+  const __bf16* src[4];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int x0 = mb * SMALL;
+    src[c] = LX == ROW ? p.x.p + (long)min(x0 + 32 * c + lr, p.x.n - 1) * p.x.ld + crow + (long)w0 * BK
+                       : p.x.p + (long)(w0 * BK + 32 * c + lr) * p.x.ld + min(x0 + ccol, p.x.n - 8);
+    if (PAIRED) {      // 32 columns of each matrix
+      src[2 + c] = (ccol < 32 ? p.w.p : p.w1) + (long)(w0 * BK + 32 * c + lr) * p.w.ld + nb * 32 + (ccol & 31);
+    } else {
+      const int n0 = nb * SMALL;
+      src[2 + c] = LW == ROW ? p.w.p + (long)min(n0 + 32 * c + lr, p.w.n - 1) * p.w.ld + crow + (long)w0 * BK
+                             : p.w.p + (long)(w0 * BK + 32 * c + lr) * p.w.ld + min(n0 + ccol, p.w.n - 8);
+    }
+  }
+  const long xstep = LX == ROW ? BK : BK * p.x.ld, wstep = LW == ROW ? BK : BK * p.w.ld;
+  int k_left = p.K - w0 * BK;      // of the window being issued
+  auto issue = [&](int slot) MM1_INLINE {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const __bf16* s = src[c];
+      if (RAGGED_K && k_left < BK && 32 * (c & 1) + lr >= k_left) s = reinterpret_cast<const __bf16*>(kZeros);
+      dma16(s, lds0 + slot * SMALL_SLOT + c * PANEL + w * 1024);
+      src[c] += c < 2 ? xstep : wstep;
+    }
+    k_left -= BK;
+  };
+  const SmallFrag<LX> fx(lane, lds0, w & 1);
+  const SmallFrag<LW> fw(lane, lds0 + 2 * PANEL, PAIRED ? 0 : w >> 1);
+  const SmallFrag<LW> fw1(lane, lds0 + 2 * PANEL, 1);     // PAIRED: the second matrix
+#pragma unroll
+  for (int a = 0; a < (PAIRED ? 2 : 1); ++a) acc[a] = zero16();
+  for (int i = 0; i < SMALL_SLOTS - 1 && i < nw; ++i) issue(i);
+  for (int i = 0; i < nw; ++i) {
+    // window i has landed; the newer ones stay in flight
+    if (i + SMALL_SLOTS - 2 < nw)
+      __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (SMALL_SLOTS - 2)) : "memory");
+    else
+      wait_dma();
+    lds_barrier();     // ... everyone's, and every read of window i - 1 is done
+    if (i + SMALL_SLOTS - 1 < nw) issue((i + SMALL_SLOTS - 1) % SMALL_SLOTS);
+    const int so = (i % SMALL_SLOTS) * SMALL_SLOT;
+    if constexpr (PAIRED) {
+      const int kk0 = 2 * (w >> 1);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const bf16x8 x = fx.get(so, kk0 + j);
+        acc[0] = mfma32(fw.get(so, kk0 + j), x, acc[0]);
+        acc[1] = mfma32(fw1.get(so, kk0 + j), x, acc[1]);
+      }
+    } else {
+      bf16x8 x[4], y[4];
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        x[kk] = fx.get(so, kk);
+        y[kk] = fw.get(so, kk);
+      }
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) acc[0] = mfma32(y[kk], x[kk], acc[0]);
+    }
+  }
+  __syncthreads();
+}
+
+// PAIRED: adds the second k half's accumulators (waves 2, 3) to the first's
+// (waves 0, 1, for which it returns true).
+__device__ __forceinline__ bool small_sum_halves(char* smem, f32x16 (&acc)[2]) {
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  f32x4* buf = reinterpret_cast<f32x4*>(smem) + (w & 1) * 512 + lane;
+  if (w >> 1) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[a][4 * q + e];
+        buf[(4 * a + q) * 64] = v;
+      }
+    }
+  }
+  __syncthreads();
+  if (w >> 1) return false;
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 v = buf[(4 * a + q) * 64];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[a][4 * q + e] += v[e];
+    }
+  }
+  return true;
+}
+
 }  // namespace gemm
 }  // namespace mm1

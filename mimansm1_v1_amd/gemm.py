@@ -29,7 +29,12 @@ def _layout(t):
     return None
 
 
-def applies(x, w) -> bool:
+# Products that mm1_gemm_estimate_us puts at this or less run on its small tiles:
+# torch's GEMM takes 21 us of host time a call, this 11 (two launches: 15).
+SMALL_US = 14.0
+
+
+def applies(x, w, small=True) -> bool:
     """Whether mm1_gemm takes x [M, K] w [N, K]^T (K a multiple of 128 unless
     both are k-major, N of 8, not x k-major with w k-contiguous) and was measured faster than
     hipBLASLt's GEMM at such a size (MI355X; T tokens, widths 1280 to 49152):
@@ -45,20 +50,24 @@ def applies(x, w) -> bool:
       331 -> 182 us); hipBLASLt is faster elsewhere (16384 x 3328 x 1280: 136
       against 143 us).
     Below, too few tiles or windows are left per CU (1792 x 1280 x 4096, both
-    k-major: 45 against 48 us)."""
+    k-major: 45 against 48 us) until the product is so small that the host's
+    work decides: those run on the small tiles (`small`, SMALL_US)."""
     m, k = x.shape
     n = w.shape[0]
-    if m * n * k < 24 * 10 ** 9:
+    if not x.is_cuda or m < 1 or n < 1 or k < 1:
+        return False
+    few = m * n * k < 24 * 10 ** 9
+    if few and not (small and 0 <= _lib.load().mm1_gemm_estimate_us(m, n, k) <= SMALL_US):
         return False
     lx, lw = _layout(x), _layout(w)
     if lx is None or lw is None or (lx[0] == COL and lw[0] == ROW):
         return False
-    if (k % 128 and lx[0] == ROW) or n % 8 or m < 1 or k < 1 or w.shape[1] != k or w.device != x.device:
+    if (k % 128 and lx[0] == ROW) or n % 8 or w.shape[1] != k or w.device != x.device:
         return False
     for (layout, ld), rows in ((lx, m), (lw, n)):
         if (256 * ld + k if layout == ROW else 64 * ld + rows) >= 1 << 30 or rows > 1 << 26:
             return False
-    if lw[0] == COL:
+    if few or lw[0] == COL:
         return True
     return (n % 320 == 0 and m * n >= 230 * 256 * 320) or (k >= 16384 and m * n >= 16 * 256 * 256)
 
@@ -94,7 +103,7 @@ def product(x, w, w1=None, out_dtype=DTYPE, split=None):
             raise ValueError("split halves the columns")
         out, out1 = (torch.empty(m, split, dtype=out_dtype, device=x.device) for _ in range(2))
     lib = _lib.load()
-    ws_bytes = lib.mm1_gemm_workspace_size(m, n, k)
+    ws_bytes = lib.mm1_gemm_workspace_size(m, n, k, int(w1 is not None))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     ptr = lambda t: None if t is None else t.data_ptr()
     rc = lib.mm1_gemm(x.data_ptr(), lx, ldx, w.data_ptr(), lw, ldw, ptr(w1), k_cut, out.data_ptr(), ptr(out1),

@@ -27,17 +27,20 @@ def check(out, x, w):
     assert over <= 0, over
 
 
-# (M, N, K): smallest; ragged rows and columns of a tile; several tiles; a
+# (M, N, K), small tiles and large: smallest; ragged rows and columns of a tile; several tiles; a
 # 320-column width; few tiles over a long K (split over all CUs, runs of one
 # and of two tiles); fewer window pairs than CUs (empty runs); 257 tiles (one left over)
 SHAPES = [(8, 8, 128), (256, 256, 128), (264, 520, 256), (776, 1288, 384), (1000, 320, 640),
-          (512, 1280, 8192), (264, 264, 16384), (8, 8, 16384), (1280, 640, 6144), (65792, 256, 256)]
+          (512, 1280, 8192), (264, 264, 16384), (8, 8, 16384), (1280, 640, 6144), (65792, 256, 256),
+          (64, 64, 128), (65, 72, 128), (128, 1792, 1280), (77, 1280, 3328), (1, 1280, 6656), (320, 1280, 1280),
+          (5000, 1288, 640), (3000, 3336, 384), (4104, 328, 896), (1288, 1288, 16384)]
 
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_products_vs_fp64(hip_device, M, N, K, layout):
     gen = torch.Generator(device=hip_device).manual_seed(M + N + K)
+    M = (M + 7) // 8 * 8 if layout == "tn" else M      # k-major operands: rows of 8
     x = operand(M, K, layout == "tn", gen, hip_device)
     w = operand(N, K, layout != "nt", gen, hip_device)
     for dtype in (torch.bfloat16, torch.float32):
@@ -72,7 +75,7 @@ def test_ragged_reduction_of_weight_gradients(hip_device, K):
     """Both operands k-major: the k rows past K, which memory may hold NaN at,
     count as zeros."""
     gen = torch.Generator(device=hip_device).manual_seed(K)
-    for M, N in ((264, 1288), (1280, 640)):
+    for M, N in ((264, 1288), (1280, 640), (3080, 3336)):
         xs, ws = (torch.full((K + 130, n), float("nan"), dtype=torch.bfloat16, device=hip_device) for n in (M, N))
         for t in (xs, ws):
             t[:K] = torch.randn(K, t.shape[1], device=hip_device, generator=gen).to(torch.bfloat16)
@@ -96,7 +99,7 @@ def test_c_abi_refuses_what_the_kernels_do_not_take(hip_device):
                 dict(M=1 << 29), dict(ldx=1 << 22)):
         assert call(**bad) == -2, bad
     assert call(x=p + 2) == -6
-    need = lib.mm1_gemm_workspace_size(512, 1280, 8192)
+    need = lib.mm1_gemm_workspace_size(512, 1280, 8192, 0)
     assert need > 0
     big = torch.zeros(1280 * 8192, dtype=torch.bfloat16, device=hip_device).data_ptr()
     assert lib.mm1_gemm(big, 0, 8192, big, 0, 8192, None, 0, big, None, 0, 1280, 0, None, 0, 512, 1280, 8192,
