@@ -40,6 +40,11 @@ int mm1_swiglu_gate_up(const void* x, const void* w_gate, const void* w_up,
                        void* gate, void* up, void* act,
                        int T, int d_model, int ffn, int mode, void* stream);
 
+/* act of mode MM1_SWIGLU_TRAIN, bitwise, without gate and up: the forward of
+ * FusedSwiGLU when no gradient is wanted. */
+int mm1_swiglu_act(const void* x, const void* w_gate, const void* w_up, void* act,
+                   int T, int d_model, int ffn, void* stream);
+
 /* SwiGLU gradient: with s = sigmoid(gate), in fp32 from the bf16 inputs,
  *   d_gate = bf16(d_act * up * s * (1 + gate * (1 - s))),  d_up = bf16(d_act * gate * s).
  * d_gate and d_up rows have stride ld_out elements (ld_out >= ffn, a multiple

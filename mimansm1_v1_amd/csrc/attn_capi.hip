@@ -592,6 +592,16 @@ int mm1_swiglu_gate_up(const void* x, const void* w_gate, const void* w_up, void
                                              static_cast<hipStream_t>(stream)));
 }
 
+int mm1_swiglu_act(const void* x, const void* w_gate, const void* w_up, void* act, int T, int d_model, int ffn,
+                   void* stream) {
+  if (!x || !w_gate || !w_up || !act) return MM1_E_NULL;
+  int rc = check_swiglu_shape(T, d_model, ffn);
+  if (rc) return rc;
+  if (!aligned16(x) || !aligned16(w_gate) || !aligned16(w_up) || !aligned16(act)) return MM1_E_ALIGN;
+  return from_hip(mm1::launch_swiglu_gate_up(x, w_gate, w_up, nullptr, nullptr, act, T, d_model, ffn, 3,
+                                             static_cast<hipStream_t>(stream)));
+}
+
 int mm1_swiglu_grad(const void* d_act, const void* gate, const void* up, void* d_gate, void* d_up,
                     int T, int ffn, long ld_out, void* stream) {
   if (!d_act || !gate || !up || !d_gate || !d_up) return MM1_E_NULL;

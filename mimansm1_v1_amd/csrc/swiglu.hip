@@ -197,7 +197,8 @@ static hipError_t launch_gate_up_t(const __bf16* x, const __bf16* wg, const __bf
 }
 
 // mode: 0 = act only, fp32 epilogue (gate_up_swiglu); 1 = gate and up only
-// (gate_up_split); 2 = gate, up and act with bf16 rounding steps (FusedSwiGLU).
+// (gate_up_split); 2 = gate, up and act with bf16 rounding steps (FusedSwiGLU);
+// 3 = that act alone (FusedSwiGLU without gradients).
 hipError_t launch_swiglu_gate_up(const void* x, const void* wg, const void* wu, void* gate, void* up,
                                  void* act, int T, int d, int F, int mode, hipStream_t stream) {
   auto xp = static_cast<const __bf16*>(x);
@@ -209,6 +210,7 @@ hipError_t launch_swiglu_gate_up(const void* x, const void* wg, const void* wu, 
   switch (mode) {
     case 0: return launch_gate_up_t<false, 1>(xp, gp, up_w, go, uo, ao, T, d, F, stream);
     case 1: return launch_gate_up_t<true, 0>(xp, gp, up_w, go, uo, ao, T, d, F, stream);
+    case 3: return launch_gate_up_t<false, 2>(xp, gp, up_w, go, uo, ao, T, d, F, stream);
     default: return launch_gate_up_t<true, 2>(xp, gp, up_w, go, uo, ao, T, d, F, stream);
   }
 }

@@ -140,6 +140,18 @@ class TrainKernel(_GateUp):
     def __call__(self, x, w_gate, w_up):
         return self.launch(x, w_gate, w_up)
 
+    def act_only(self, x, w_gate, w_up):
+        """The act of a call, bitwise, without writing gate and up."""
+        T, d, Fh = self.shape
+        _require(x, "x", (T, d))
+        _require(w_gate, "w_gate", (d, Fh))
+        _require(w_up, "w_up", (d, Fh))
+        act = torch.empty(T, Fh, dtype=DTYPE, device=x.device)
+        rc = _lib.load().mm1_swiglu_act(x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), act.data_ptr(), T, d, Fh,
+                                        _stream(x.device))
+        _lib.check(rc, "mm1_swiglu_act")
+        return act
+
 
 class GradKernel:
     """swiglu_grad (SW:202-240): (d_act, gate, up) -> (d_gate, d_up).  With
@@ -207,6 +219,14 @@ def _matmul(x, w):
     return gemm.product(x, w) if gemm.applies(x, w) else x @ w.t()
 
 
+def _forward_only(x, w_gate, w_up, w_down):
+    """FusedSwiGLU's output, bitwise, where no backward follows: gate and up stay
+    in registers (16384 tokens, 1280 x 3328: 218 MB less written, 372 -> 345 us;
+    1000 tokens 57 -> 55)."""
+    kernel = get_kernel("train", x.shape[0], x.shape[1], w_gate.shape[1])
+    return _matmul(kernel.act_only(x, w_gate, w_up), w_down.t())
+
+
 class FusedSwiGLU(torch.autograd.Function):
     """Same signature and returns as SW:276-301.  Forward: one HIP launch for
     gate, up and act (the reference's split kernel plus its two elementwise
@@ -221,6 +241,8 @@ class FusedSwiGLU(torch.autograd.Function):
     def forward(ctx, x, w_gate, w_up, w_down):
         tokens, d_model = x.shape
         ffn = w_gate.shape[1]
+        if not any(ctx.needs_input_grad):
+            return _forward_only(x, w_gate, w_up, w_down)
         gate, up, act = get_kernel("train", tokens, d_model, ffn)(x, w_gate, w_up)
         out = _matmul(act, w_down.t())
         ctx.save_for_backward(x, w_gate, w_up, w_down, gate, up, act)
@@ -252,8 +274,18 @@ class FusedSwiGLU(torch.autograd.Function):
         return d_x, d_w_gate, d_w_up, d_w_down
 
 
+class _FusedSwiGLUNoGrad(torch.autograd.Function):
+    """FusedSwiGLU under no_grad, where needs_input_grad of a parameter is still
+    true.  A Function, so that transforms refuse it as they refuse FusedSwiGLU."""
+
+    @staticmethod
+    def forward(ctx, x, w_gate, w_up, w_down):
+        return _forward_only(x, w_gate, w_up, w_down)
+
+
 def fused_swiglu(x, w_gate, w_up, w_down):
-    return FusedSwiGLU.apply(x, w_gate, w_up, w_down)
+    function = FusedSwiGLU if torch.is_grad_enabled() else _FusedSwiGLUNoGrad
+    return function.apply(x, w_gate, w_up, w_down)
 
 
 @dataclass

@@ -155,17 +155,24 @@ def test_swiglu_deterministic(hip_device):
 
 @pytest.mark.parametrize("T", [1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 256, 320, 333])
 @pytest.mark.parametrize("d,Fh", [(128, 128), (256, 640), (1280, 3328)])
-def test_few_tokens(hip_device, T, d, Fh):
+def test_few_tokens_and_the_act_alone(hip_device, T, d, Fh):
     """The small tiles at the edges of their 64 tokens and 32 columns, on either
     side of the switch to the large ones: gate and up within half a bf16 ulp of
     the exact products plus fp32 rounding of the sums, the training mode's
-    gate and up bitwise those of split mode."""
+    three outputs bitwise those of split mode and of the act-only call."""
     from mimansm1_v1_amd import swiglu as S
     gen = torch.Generator(device=hip_device).manual_seed(T)
     x = torch.randn(T, d, device=hip_device, generator=gen).to(torch.bfloat16)
     wg, wu = ((torch.randn(d, Fh, device=hip_device, generator=gen) * 0.05).to(torch.bfloat16) for _ in range(2))
-    gate, up, _ = S.get_kernel("train", T, d, Fh)(x, wg, wu)
+    gate, up, act = S.get_kernel("train", T, d, Fh)(x, wg, wu)
     for got, w in ((gate, wg), (up, wu)):
         exact, size = x.double() @ w.double(), x.double().abs() @ w.double().abs()
         assert ((got.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + d * 2.0 ** -24 * size).all()
     assert all(torch.equal(a, b) for a, b in zip((gate, up), S.get_kernel("split", T, d, Fh)(x, wg, wu)))
+    assert torch.equal(act, S.get_kernel("train", T, d, Fh).act_only(x, wg, wu))
+    w_down = wg.t().contiguous()
+    out = S.fused_swiglu(x, wg, wu, w_down)                       # nothing needs a gradient
+    kept = S.fused_swiglu(x.requires_grad_(True), wg, wu, w_down)
+    with torch.no_grad():
+        assert torch.equal(out, S.fused_swiglu(x, wg, wu, w_down))
+    assert torch.equal(out, kept.detach()) and kept.requires_grad and not out.requires_grad
