@@ -104,3 +104,22 @@ def test_c_abi_refuses_what_the_kernels_do_not_take(hip_device):
     big = torch.zeros(1280 * 8192, dtype=torch.bfloat16, device=hip_device).data_ptr()
     assert lib.mm1_gemm(big, 0, 8192, big, 0, 8192, None, 0, big, None, 0, 1280, 0, None, 0, 512, 1280, 8192,
                         None) == -4
+
+
+@pytest.mark.parametrize("sizes", [(8, 0, 0, 0), (0, 24, 0, 8), (2048, 8, 2056, 0), (16, 1280 * 1280, 40, 1 << 20)])
+def test_cast_of_several_tensors(hip_device, sizes):
+    """One launch rounds the fp32 tensors to bf16 as torch does, specials
+    included, one after the other."""
+    src = [torch.randn(n, device=hip_device) * 3 for n in sizes]
+    for t in src:
+        if t.numel():
+            t[:8] = torch.tensor([float("inf"), -float("inf"), float("nan"), 0.0, -0.0, 1e-40, 3.3895e38, 1.00390625])
+    dst = torch.empty(sum(sizes), dtype=torch.bfloat16, device=hip_device)
+    segments = [a for t in src for a in (t.data_ptr() if t.numel() else None, t.numel())]
+    stream = torch.cuda.current_stream().cuda_stream
+    lib = _lib.load()
+    assert lib.mm1_cast_bf16(*segments, dst.data_ptr(), stream) == 0
+    torch.testing.assert_close(dst, torch.cat(src).to(torch.bfloat16), rtol=0, atol=0, equal_nan=True)
+    p = dst.data_ptr()
+    for bad in ((None, 8), (p, 4), (p, -8), (p + 4, 8)):
+        assert lib.mm1_cast_bf16(*bad, *segments[2:], dst.data_ptr(), stream) < 0, bad
