@@ -479,7 +479,7 @@ def time_sublayer(batch, seq, device, steps, warmup):
     under bf16 autocast, x ~ N(0,1), weights ~ N(0, 0.02^2).  Besides the whole
     step, its parts are timed on the same tensors: the attention kernels (fwd +
     bwd), the projection GEMMs (QKV and wo, fwd + both backward products, as
-    BF16Linear runs them on hipBLASLt) and the QK-norm + RoPE kernels (fwd +
+    BF16Linear runs them) and the QK-norm + RoPE kernels (fwd +
     bwd)."""
     import torch
     import torch.nn.functional as F
@@ -570,8 +570,8 @@ def time_sublayer(batch, seq, device, steps, warmup):
         "gemm_tflops": round(gemm_flops / (parts["gemm"] * 1e-3) / 1e12, 2),
         "flops": {"attention": attn_flops, "gemm": gemm_flops},
         "note": "bf16 autocast; attention = flash_attention fwd+bwd kernels, gemm = QKV (1280->1792) and "
-                "wo (1280->1280) fwd + dX + dW as the step runs them (BF16Linear: hipBLASLt GEMMs, dW over 8 "
-                "token chunks with fp32 outputs), qknorm_rope = fwd+bwd kernels; "
+                "wo (1280->1280) fwd + dX + dW as the step runs them (BF16Linear: the GEMM core or "
+                "hipBLASLt by size, dW with fp32 outputs), qknorm_rope = fwd+bwd kernels; "
                 "other = casts, weight concatenation and autograd bookkeeping of the whole step",
     }
 
