@@ -249,7 +249,9 @@ class TiedCrossEntropy(torch.autograd.Function):
     def forward(ctx, hidden, embedding, targets, chunk):
         tokens, d_model = hidden.shape
         vocab = embedding.shape[0]
-        weight = embedding.to(DTYPE).contiguous()
+        # a copy in every dtype: the backward's matrix stays the forward's when the
+        # embedding changes in between, and the kernels take any embedding's alignment
+        weight = embedding.to(DTYPE, copy=True, memory_format=torch.contiguous_format)
         _check_bf16_hip(hidden, weight)
         kernel = get_kernel((tokens, d_model, vocab))
         targets = targets.contiguous()

@@ -154,3 +154,27 @@ def test_tied_head_reads_the_embedding_by_rows(hip_device, T, V, chunk, dtype):
     for a, b in ((hid.grad, rows.grad), (emb.weight.grad, wd.grad.t())):
         a, b = a.double(), b.double()
         assert (a - b).norm() <= 2.0 ** -8 * b.norm()
+
+
+@pytest.mark.parametrize("chunk", [1024, 256])
+def test_tied_head_holds_its_own_bf16_matrix(hip_device, chunk):
+    """A bf16 embedding at an address that is no multiple of 16 bytes, changed
+    between forward and backward: the loss and every gradient are bitwise those
+    of an aligned embedding left alone."""
+    from mimansm1_v1_amd import lm_head as L
+    T, V = 130, 1024
+    h, w, t = (x.to(hip_device) for x in LMO.make_inputs(T, 1280, V, seed=3, n_ignore=5))
+    flat = torch.empty(V * 1280 + 1, dtype=torch.bfloat16, device=hip_device)
+    results = []
+    for weight, change in ((w.t().contiguous().bfloat16(), False),
+                           (flat[1:].view(V, 1280).copy_(w.t()), True)):
+        emb = torch.nn.Embedding(V, 1280, _weight=weight)
+        head = L.LMHead(L.HeadConfig(vocab=V, logit_scale=1.0, chunk=chunk), emb)
+        hid = h.clone().requires_grad_(True)
+        loss = head(hid, t)
+        if change:
+            with torch.no_grad():
+                emb.weight.add_(1.0)
+        loss.backward()
+        results.append((loss.detach(), hid.grad, emb.weight.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
