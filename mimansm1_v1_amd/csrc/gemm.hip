@@ -51,13 +51,11 @@ __device__ __forceinline__ void store_rows32(const Output& o, char* lds, int lan
   };
   if constexpr (F32) {
 #pragma unroll
-    for (int b = 0; b < S::TJ; ++b) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float* p = out_at<float>(o, row0 + (lane & 31), col0 + 32 * b + 8 * q + 4 * (lane >> 5));
-        if (p) *reinterpret_cast<f32x4*>(p) = val(b, q);
-      }
-    }
+    for (int b = 0; b < S::TJ; ++b)
+      gemm::store_block_f32<S::STAGE_BYTES / 128, NT>(
+          lds, lane, [&](int q) { return val(b, q); },
+          [&](int r) { return out_at<float>(o, row0 + r, col0 + 32 * b); },
+          [&](int c) { return col0 + 32 * b + 4 * c < o.N; });
   } else if constexpr (S::TJ == 2) {
     gemm::store_block128<NT>(
         lds, lane, bf16_quad, [&](int r) { return out_at<__bf16>(o, row0 + r, col0); },
@@ -77,11 +75,9 @@ __device__ __forceinline__ void store_rows32(const Output& o, char* lds, int lan
 template <bool F32, class Val>
 __device__ __forceinline__ void store_block32(const Output& o, char* lds, int lane, long row0, int col0, Val&& val) {
   if constexpr (F32) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float* p = out_at<float>(o, row0 + (lane & 31), col0 + 8 * q + 4 * (lane >> 5));
-      if (p) *reinterpret_cast<f32x4*>(p) = val(q);
-    }
+    gemm::store_block_f32<16, false>(
+        lds, lane, val, [&](int r) { return out_at<float>(o, row0 + r, col0); },
+        [&](int c) { return col0 + 4 * c < o.N; });
   } else {
     gemm::store_block64<false>(
         lds, lane,
@@ -364,8 +360,9 @@ hipError_t launch_small(const Launch& l) {
 
 template <class S>
 hipError_t launch_o(const Launch& l) {
-  if (l.a.f32) return launch_s<S, true, false>(l);
-  return (long)l.a.M * l.a.N * 2 > gemm::CACHED_BYTES ? launch_s<S, false, true>(l) : launch_s<S, false, false>(l);
+  const bool nt = (long)l.a.M * l.a.N * (l.a.f32 ? 4 : 2) > gemm::CACHED_BYTES;
+  if (l.a.f32) return nt ? launch_s<S, true, true>(l) : launch_s<S, true, false>(l);
+  return nt ? launch_s<S, false, true>(l) : launch_s<S, false, false>(l);
 }
 
 }  // namespace
