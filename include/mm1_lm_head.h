@@ -56,7 +56,8 @@ int mm1_lm_head_dlogits(const void* hidden, const void* weight, const long long*
                         int T, int d_model, int vocab, int v0, int vn, void* stream);
 
 /* The same two calls for a weight stored [vocab, d_model] (an embedding
- * matrix as it lies in memory: a head tied to it needs no transposed copy). */
+ * matrix as it lies in memory: a head tied to it needs no transposed copy).
+ * Here the bytes of 256 rows of the weight must be below 2^31 (MM1_E_SHAPE). */
 int mm1_lm_head_lse_rows(const void* hidden, const void* weight, const long long* targets, long long ignore_index,
                          float* lse, float* target_logit, float* loss, void* workspace, size_t workspace_bytes,
                          int T, int d_model, int vocab, void* stream);

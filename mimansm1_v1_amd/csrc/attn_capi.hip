@@ -615,9 +615,14 @@ int mm1_swiglu_grad(const void* d_act, const void* gate, const void* up, void* d
 
 static int check_lm_shape(int T, int d, int V) {
   if (T < 1 || (long)T > kMaxTokens || d < 128 || d % 128 != 0 || V < 128 || V % 128 != 0) return MM1_E_SHAPE;
-  // 32-bit byte offsets inside hidden and a 64-row slab of the weight
+  // 32-bit byte offsets inside hidden and a 64-row slab of a [d, V] weight
   if ((long)T * d >= (1L << 30) || 64L * V >= (1L << 30)) return MM1_E_SHAPE;
   return MM1_OK;
+}
+
+// Of a [V, d] weight a tile's copies span 256 rows of d.
+static int check_lm_rows(bool vocab_rows, int d, int V) {
+  return vocab_rows && !mm1::gemm_operand_fits(MM1_GEMM_ROW, d, V, d) ? MM1_E_SHAPE : MM1_OK;
 }
 
 size_t mm1_lm_head_workspace_size(int T, int vocab) {
@@ -631,6 +636,7 @@ static int lm_head_lse(const void* hidden, const void* weight, bool vocab_rows, 
   if (!hidden || !weight || !lse) return MM1_E_NULL;
   if (!targets && (target_logit || loss)) return MM1_E_NULL;
   int rc = check_lm_shape(T, d_model, vocab);
+  if (!rc) rc = check_lm_rows(vocab_rows, d_model, vocab);
   if (rc) return rc;
   if (!workspace || workspace_bytes < mm1::lm_head_workspace_bytes(T, vocab)) return MM1_E_WORKSPACE;
   if (!aligned16(hidden) || !aligned16(weight) || !aligned16(workspace)) return MM1_E_ALIGN;
@@ -657,6 +663,7 @@ static int lm_head_dlogits(const void* hidden, const void* weight, bool vocab_ro
                            int T, int d_model, int vocab, int v0, int vn, void* stream) {
   if (!hidden || !weight || !targets || !lse || !scale || !d_logits) return MM1_E_NULL;
   int rc = check_lm_shape(T, d_model, vocab);
+  if (!rc) rc = check_lm_rows(vocab_rows, d_model, vocab);
   if (rc) return rc;
   if (v0 < 0 || vn < 128 || v0 % 128 != 0 || vn % 128 != 0 || (long)v0 + vn > vocab || ld < vn || ld % 8 != 0)
     return MM1_E_SHAPE;

@@ -238,6 +238,12 @@ class FusedCrossEntropy(torch.autograd.Function):
         return d_hidden.to(hidden.dtype), d_weight, None, None
 
 
+def rows_apply(d_model) -> bool:
+    """Whether the kernels read a [V, d_model] matrix by rows: the copies of a
+    tile span 256 of its rows, whose byte offsets are 32-bit."""
+    return 257 * d_model < 1 << 30
+
+
 class TiedCrossEntropy(torch.autograd.Function):
     """FusedCrossEntropy for a head tied to its embedding: `embedding` is the
     [V, d] matrix as it lies in memory, which the kernels read by rows, so no
@@ -333,8 +339,9 @@ class LMHead(nn.Module):
 
     def _loss_hip(self, rows, weight, targets):
         # bf16 kernels: the fp32 stream and matrix become contiguous bf16 here
-        # (LM:313-323); a tied matrix is read in the embedding's own layout
-        if self.cfg.tied:
+        # (LM:313-323); a tied matrix is read in the embedding's own layout, or,
+        # in widths beyond that kernel's offsets, from its transposed copy
+        if self.cfg.tied and rows_apply(self.cfg.d_model):
             return TiedCrossEntropy.apply(rows.to(DTYPE).contiguous(), self.embedding[0].weight, targets,
                                           self.cfg.chunk)
         return fused_cross_entropy(rows.to(DTYPE).contiguous(), weight.to(DTYPE).contiguous(), targets,

@@ -385,6 +385,21 @@ def test_lm_head_argument_errors_without_device(lib):
     assert dl(out=FAKE + 8) == -6
 
 
+@pytest.mark.parametrize("d,fits", [(1280, True), ((1 << 30) // 257 // 128 * 128, True), (1 << 22, False),
+                                    (16909440, False), (1 << 25, False)])
+def test_lm_head_rows_entries_bound_the_width(lib, d, fits):
+    """A [V, d] weight whose 256-row offsets pass 32 bits is refused (what fits
+    gets as far as the next check); the [d, V] entries take every such width."""
+    from mimansm1_v1_amd import lm_head as L
+    rest = (FAKE, -100, FAKE, FAKE, FAKE, None, 0, 1, d, 384, None)
+    assert lib.mm1_lm_head_lse_rows(FAKE, FAKE, *rest) == (-4 if fits else -2)
+    assert lib.mm1_lm_head_lse(FAKE, FAKE, *rest) == -4
+    rest = (FAKE, -100, FAKE, FAKE, FAKE + 8, 384, 1, d, 384, 0, 384, None)
+    assert lib.mm1_lm_head_dlogits_rows(FAKE, FAKE, *rest) == (-6 if fits else -2)
+    assert lib.mm1_lm_head_dlogits(FAKE, FAKE, *rest) == -6
+    assert L.rows_apply(d) is fits
+
+
 # ---------------------------------------------------------------------------
 # Workgroup dispatch order of the causal grids (host-side model, no device).
 

@@ -345,3 +345,23 @@ def test_bench_select_tiles_follows_the_record(monkeypatch):
     monkeypatch.setattr(A, "OVERLAP_DQ", False)
     assert bench.select_tiles(2, 8192)["overlap"] is False
     assert bench.select_tiles(2, 8192, "1,5,0") == {"fwd": 1, "dkdv": 5, "dq": 0, "overlap": False}
+
+
+@pytest.mark.parametrize("d", [1280, 1 << 22, 16909440])
+def test_tied_head_wide_embeddings_go_through_the_transposed_copy(monkeypatch, d):
+    """Widths that the row-reading kernels refuse take the [d, V] kernels, as an
+    untied head does; all others read the embedding by rows."""
+    from mimansm1_v1_amd import lm_head as L
+    calls = []
+    monkeypatch.setattr(L, "fused_cross_entropy", lambda h, w, t, chunk: calls.append(("columns", h, w, chunk)))
+    monkeypatch.setattr(L.TiedCrossEntropy, "apply", lambda h, e, t, chunk: calls.append(("rows", h, e, chunk)))
+    with torch.device("meta"):
+        emb = torch.nn.Embedding(384, d)
+        head = L.LMHead(L.HeadConfig(d_model=d, vocab=384, chunk=128), emb)
+        head(torch.empty(2, d), torch.zeros(2, dtype=torch.int64))
+    (kind, hidden, weight, chunk), = calls
+    assert kind == ("rows" if d == 1280 else "columns") and chunk == 128
+    assert hidden.shape == (2, d) and hidden.dtype == torch.bfloat16
+    assert tuple(weight.shape) == ((384, d) if kind == "rows" else (d, 384))
+    if kind == "columns":
+        assert weight.dtype == torch.bfloat16 and weight.is_contiguous()
