@@ -168,9 +168,18 @@ __host__ __device__ inline int windows_of(int K) { return (K + 2 * BK - 1) / (2 
 __device__ __attribute__((aligned(16))) static const uint32_t kZeros[4] = {0, 0, 0, 0};
 
 // The host's bound on the copies' 32-bit byte offsets from a tile's base.
+constexpr long SPAN = 1L << 30;            // elements
 inline bool offsets_fit(Layout l, long ld, int n, int K) {
-  return l == ROW ? BM * ld + K < (1L << 30) : BK * ld + n < (1L << 30);
+  return l == ROW ? BM * ld + K < SPAN : BK * ld + n < SPAN;
 }
+
+// Byte offset of element k of row `row` of a ROW operand, unsigned: a tile's W
+// has up to Wide320::BN rows, which at the longest stride pass 2^31.
+__host__ __device__ constexpr uint32_t row_off(int row, long ld, int k) {
+  return (uint32_t)row * (uint32_t)(2 * ld) + (uint32_t)(2 * k);
+}
+constexpr long LD_MAX = SPAN / BM - 8;     // the longest stride that fits
+static_assert(row_off(Wide320::BN - 1, LD_MAX, BK) == 2 * ((Wide320::BN - 1) * LD_MAX + BK), "offsets of the widest tile");
 
 __device__ __forceinline__ void tile_coords(int t, int n_mblk, int n_nblk, int& mb, int& nb) {
   const int per_group = GROUP * n_nblk;
@@ -322,7 +331,7 @@ __device__ __forceinline__ void run(const Problem& p, char* smem, Pro&& pro, Epi
   // copy n of an operand in a tile that crosses its edge (`room` >= 1)
   auto edge_off = [&](auto layout, int n, int room, long ld) MM1_INLINE {
     if constexpr (decltype(layout)::value == ROW)
-      return (uint32_t)(min(prow + 64 * n, room - 1) * (int)(2 * ld) + 2 * crow);
+      return row_off(min(prow + 64 * n, room - 1), ld, crow);
     else
       return (uint32_t)(prow * (int)(2 * ld) + 2 * min(64 * n + ccol, room - 8));
   };
