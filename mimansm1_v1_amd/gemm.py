@@ -29,6 +29,12 @@ def _layout(t):
     return None
 
 
+def recorded(*tensors) -> bool:
+    """Whether autograd records an operation on these (a backward under
+    create_graph): the kernels' products leave no graph, torch's do."""
+    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+
+
 # Products that mm1_gemm_estimate_us puts at this or less run on its small tiles:
 # torch's GEMM takes 21 us of host time a call, this 11 (two launches: 15).
 SMALL_US = 14.0
@@ -54,7 +60,7 @@ def applies(x, w, small=True) -> bool:
     work decides: those run on the small tiles (`small`, SMALL_US)."""
     m, k = x.shape
     n = w.shape[0]
-    if not x.is_cuda or m < 1 or n < 1 or k < 1:
+    if not x.is_cuda or m < 1 or n < 1 or k < 1 or recorded(x, w):
         return False
     few = m * n * k < 24 * 10 ** 9
     if few and not (small and 0 <= _lib.load().mm1_gemm_estimate_us(m, n, k) <= SMALL_US):
@@ -77,7 +83,7 @@ def applies_joined(x, w, w1) -> bool:
     k = w.shape[1]
     if x.shape[0] * w.shape[0] * 2 * k < 24 * 10 ** 9:
         return False
-    return (_layout(w) is not None and _layout(w) == _layout(w1) and w.shape == w1.shape
+    return (_layout(w) is not None and _layout(w) == _layout(w1) and w.shape == w1.shape and not recorded(w1)
             and k % 128 == 0 and x.shape[1] == 2 * k and applies(x[:, :k], w))
 
 

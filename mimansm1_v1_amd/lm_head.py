@@ -179,7 +179,9 @@ def _matmul(x, w, out_dtype=DTYPE):
     """x w^T on the GEMM core where it applies (gemm.py), else torch's GEMM."""
     if gemm.applies(x, w):
         return gemm.product(x, w, out_dtype=out_dtype)
-    return x @ w.t() if out_dtype == DTYPE else torch.mm(x, w.t(), out_dtype=out_dtype)
+    if out_dtype == DTYPE or gemm.recorded(x, w):       # mm with an out_dtype has no derivative
+        return (x @ w.t()).to(out_dtype)
+    return torch.mm(x, w.t(), out_dtype=out_dtype)
 
 
 def _check_bf16_hip(hidden, weight):
@@ -249,15 +251,14 @@ class TiedCrossEntropy(torch.autograd.Function):
     [V, d] matrix as it lies in memory, which the kernels read by rows, so no
     transposed copy is made (at V 49152, d 1280 the transpose alone took 255
     us), and its gradient leaves the product in the embedding's own layout and
-    dtype (fp32 sums, rounded once or not at all)."""
+    dtype (fp32 sums, rounded once or not at all).  `weight` is the embedding's
+    bf16 copy, an input of its own so that a recorded backward's d_hidden
+    stays connected to the embedding; its gradient goes to `embedding`."""
 
     @staticmethod
-    def forward(ctx, hidden, embedding, targets, chunk):
+    def forward(ctx, hidden, embedding, weight, targets, chunk):
         tokens, d_model = hidden.shape
         vocab = embedding.shape[0]
-        # a copy in every dtype: the backward's matrix stays the forward's when the
-        # embedding changes in between, and the kernels take any embedding's alignment
-        weight = embedding.to(DTYPE, copy=True, memory_format=torch.contiguous_format)
         _check_bf16_hip(hidden, weight)
         kernel = get_kernel((tokens, d_model, vocab))
         targets = targets.contiguous()
@@ -279,7 +280,7 @@ class TiedCrossEntropy(torch.autograd.Function):
         if chunk >= vocab:
             dl = kernel.dlogits_rows(hidden, weight, targets, lse, scale, 0, vocab)
             d_weight = _matmul(dl.t(), hidden.t(), wide).to(ctx.grad_dtype) if ctx.needs_input_grad[1] else None
-            return _matmul(dl, weight.t()), d_weight, None, None
+            return _matmul(dl, weight.t()), d_weight, None, None, None
         d_weight = torch.empty(vocab, d_model, dtype=ctx.grad_dtype, device=hidden.device)
         d_hidden = torch.zeros(tokens, d_model, dtype=torch.float32, device=hidden.device)
         for start in range(0, vocab, chunk):
@@ -287,7 +288,14 @@ class TiedCrossEntropy(torch.autograd.Function):
             dl = kernel.dlogits_rows(hidden, weight, targets, lse, scale, start, stop - start)
             d_hidden += _matmul(dl, weight[start:stop].t()).float()
             d_weight[start:stop] = _matmul(dl.t(), hidden.t(), wide)
-        return d_hidden.to(hidden.dtype), d_weight, None, None
+        return d_hidden.to(hidden.dtype), d_weight, None, None, None
+
+
+def tied_cross_entropy(hidden, embedding, targets, chunk=VOCAB_CHUNK):
+    # a copy in every dtype: the backward's matrix stays the forward's when the
+    # embedding changes in between, and the kernels take any embedding's alignment
+    weight = embedding.to(DTYPE, copy=True, memory_format=torch.contiguous_format)
+    return TiedCrossEntropy.apply(hidden, embedding, weight, targets, chunk)
 
 
 def fused_cross_entropy(hidden, weight, targets, chunk=VOCAB_CHUNK):
@@ -342,8 +350,8 @@ class LMHead(nn.Module):
         # (LM:313-323); a tied matrix is read in the embedding's own layout, or,
         # in widths beyond that kernel's offsets, from its transposed copy
         if self.cfg.tied and rows_apply(self.cfg.d_model):
-            return TiedCrossEntropy.apply(rows.to(DTYPE).contiguous(), self.embedding[0].weight, targets,
-                                          self.cfg.chunk)
+            return tied_cross_entropy(rows.to(DTYPE).contiguous(), self.embedding[0].weight, targets,
+                                      self.cfg.chunk)
         return fused_cross_entropy(rows.to(DTYPE).contiguous(), weight.to(DTYPE).contiguous(), targets,
                                    self.cfg.chunk)
 

@@ -123,3 +123,77 @@ def test_cast_of_several_tensors(hip_device, sizes):
     p = dst.data_ptr()
     for bad in ((None, 8), (p, 4), (p, -8), (p + 4, 8)):
         assert lib.mm1_cast_bf16(*bad, *segments[2:], dst.data_ptr(), stream) < 0, bad
+
+
+def _second_derivatives(call, leaves, grad_out):
+    """For each recorded first gradient of call(): None (no graph), the message
+    of torch's refusal (mm with an out_dtype has no derivative), or the gradients
+    of its sum of squares with respect to every leaf and grad_out."""
+    first = torch.autograd.grad(call(), leaves, grad_out, create_graph=True)
+    every, res = [*leaves, grad_out], []
+    for g in first:
+        try:
+            res.append(torch.autograd.grad(g.float().square().sum(), every, retain_graph=True, allow_unused=True)
+                       if g.requires_grad else None)
+        except RuntimeError as exc:
+            res.append(str(exc))
+    return res
+
+
+def _same_terms(got, want):
+    assert [type(a) for a in got] == [type(b) for b in want]
+    for a, b in zip(got, want):
+        if not isinstance(b, tuple):
+            assert a == b
+            continue
+        assert [p is None for p in a] == [q is None for q in b]
+        for p, q in zip(a, b):
+            assert q is None or (p.double() - q.double()).norm() <= 2.0 ** -6 * q.double().norm()
+
+
+def _leaf(gen, *shape, std=1.0, dtype=torch.bfloat16):
+    return (torch.randn(*shape, device=gen.device, generator=gen) * std).to(dtype).requires_grad_(True)
+
+
+@pytest.mark.parametrize("which", ["linear", "swiglu"])
+def test_recorded_backward_keeps_its_graph(hip_device, which, monkeypatch):
+    """Under create_graph the backward's products are torch's at a size that the
+    core takes too: the same terms of a second derivative, to rounding, as with
+    torch's products alone.  (64 tokens: below the batched weight gradient.)"""
+    from mimansm1_v1_amd import attention as A, swiglu as S
+    gen = torch.Generator(device=hip_device).manual_seed(3)
+    x, dy = _leaf(gen, 64, 1280), _leaf(gen, 64, 1280)
+    if which == "linear":
+        leaves = [x, _leaf(gen, 1280, 1280, std=0.02, dtype=torch.float32)]
+        call = lambda: A.BF16Linear.apply(*leaves)
+    else:
+        leaves = [x, *(_leaf(gen, *s, std=0.02) for s in ((1280, 3328), (1280, 3328), (3328, 1280)))]
+        call = lambda: S.fused_swiglu(*leaves)
+    with torch.no_grad():
+        assert gemm.applies(dy, _leaf(gen, 1280, 1280).t())
+    got = _second_derivatives(call, leaves, dy)
+    monkeypatch.setattr(gemm, "applies", lambda *a, **k: False)
+    want = _second_derivatives(call, leaves, dy)
+    assert any(isinstance(g, tuple) for g in want)
+    _same_terms(got, want)
+
+
+@pytest.mark.parametrize("T", [64, 4096])
+def test_recorded_backward_of_the_head(hip_device, T, monkeypatch):
+    """The same for the head, and for the tied head as through a transposed copy
+    of its embedding."""
+    from mimansm1_v1_amd import lm_head as L
+    gen = torch.Generator(device=hip_device).manual_seed(T)
+    h, emb = _leaf(gen, T, 1280, std=0.03), _leaf(gen, 8192, 1280, dtype=torch.float32)
+    weight = emb.detach().t().bfloat16().contiguous().requires_grad_(True)
+    gl = torch.ones((), device=hip_device, requires_grad=True)
+    t = torch.randint(0, 8192, (T,), device=hip_device, generator=gen)
+    got = _second_derivatives(lambda: L.fused_cross_entropy(h, weight, t), [h, weight], gl)
+    tied = _second_derivatives(lambda: L.tied_cross_entropy(h, emb, t), [h, emb], gl)
+    monkeypatch.setattr(gemm, "applies", lambda *a, **k: False)
+    want = _second_derivatives(lambda: L.fused_cross_entropy(h, weight, t), [h, weight], gl)
+    copied = _second_derivatives(
+        lambda: L.fused_cross_entropy(h, emb.to(torch.bfloat16).t().contiguous(), t), [h, emb], gl)
+    assert any(isinstance(g, tuple) for g in want)
+    _same_terms(got, want)
+    _same_terms(tied, copied)

@@ -354,7 +354,7 @@ def test_tied_head_wide_embeddings_go_through_the_transposed_copy(monkeypatch, d
     from mimansm1_v1_amd import lm_head as L
     calls = []
     monkeypatch.setattr(L, "fused_cross_entropy", lambda h, w, t, chunk: calls.append(("columns", h, w, chunk)))
-    monkeypatch.setattr(L.TiedCrossEntropy, "apply", lambda h, e, t, chunk: calls.append(("rows", h, e, chunk)))
+    monkeypatch.setattr(L, "tied_cross_entropy", lambda h, e, t, chunk: calls.append(("rows", h, e, chunk)))
     with torch.device("meta"):
         emb = torch.nn.Embedding(384, d)
         head = L.LMHead(L.HeadConfig(d_model=d, vocab=384, chunk=128), emb)
