@@ -24,6 +24,7 @@ another implementation.
 """
 from __future__ import annotations
 
+import hashlib
 import math
 import os
 import sys
@@ -82,6 +83,14 @@ def bwd_configs(dim=128):
         return []
     return [{**{f"dkdv_{k}": v for k, v in a.items()}, **{f"dq_{k}": v for k, v in b.items()}}
             for a in tile_space("dkdv") for b in tile_space("dq")]
+
+
+def tile_space_id(kind):
+    """Names the set of tilings that a search for `kind` ("fwd" or "bwd") chooses
+    from, whatever their order: what a tile record says it was chosen from."""
+    parts = ("fwd",) if kind == "fwd" else ("dkdv", "dq")
+    tilings = [sorted(sorted(c.items()) for c in tile_space(part)) for part in parts]
+    return hashlib.sha1(repr(tilings).encode()).hexdigest()[:12]
 
 
 def tile_index(kind, config):
@@ -399,7 +408,8 @@ def get_kernel(kind, *shape):
     reference: the tile record for this device and shape, then a timed search
     over the compiled tilings when AUTOTUNE is set and a GPU is present (its
     winner is recorded), else the defaults.  A record naming a tiling this
-    build does not have is ignored."""
+    build does not have is ignored, and, where a search can run, one that was
+    chosen from another set of tilings than this build's."""
     if kind not in ("fwd", "bwd"):
         raise ValueError(f"unknown kernel kind {kind!r}")
     key = (kind, tuple(shape), AUTOTUNE)
@@ -407,15 +417,16 @@ def get_kernel(kind, *shape):
         cls = FwdKernel if kind == "fwd" else BwdKernel
         name = f"attention_{kind}"
         kernel = None
-        remembered = tuned.lookup(name, shape)
+        search, space = AUTOTUNE and torch.cuda.is_available(), tile_space_id(kind)
+        remembered = tuned.lookup(name, shape, space=space if search else None)
         if remembered is not None and tile_index(kind, remembered) is not None:
             kernel = cls(shape, remembered)
-        elif AUTOTUNE and torch.cuda.is_available():
+        elif search:
             cls(shape, FWD_TILES if kind == "fwd" else BWD_TILES)   # shape check first
             config, latency, _ = autotune(kind, shape)
             kernel = cls(shape, config)
             kernel.latency = latency
-            tuned.record(name, shape, tuned.config_of(kernel))
+            tuned.record(name, shape, tuned.config_of(kernel), space=space)
         else:
             kernel = cls(shape, FWD_TILES if kind == "fwd" else BWD_TILES)
         _kernels[key] = kernel
@@ -1036,7 +1047,7 @@ def tune(batch=8, seq_len=2048):
     winners = {}
     for kind in spaces:
         config, latency, _ = autotune(kind, shape, verbose=True)
-        tuned.record(f"attention_{kind}", shape, config)
+        tuned.record(f"attention_{kind}", shape, config, space=tile_space_id(kind))
         _kernels.pop((kind, shape, AUTOTUNE), None)
         winners[kind] = (config, latency)
         print(f"{kind} winner {latency:.3f} ms: {config}")

@@ -53,15 +53,22 @@ def jobs(micro_batch, seq_len, cfg):
     return [("attention_fwd", "fwd", shape), ("attention_bwd", "bwd", shape)]
 
 
+def space_of(name):
+    """The tilings that a search for this job chooses from (attention.tile_space_id)."""
+    from . import attention
+    return attention.tile_space_id(name.removeprefix("attention_"))
+
+
 def tune_all(micro_batch, seq_len, cfg, force=False, store=None, lookup=None, search=None,
              record=None, out=print):
     """Tune each job of one shape; returns {name: (config, ms) or None}.  The
     lookup / search / record hooks default to the tile store and the GPU
     search; they are parameters so the control flow runs without a GPU."""
     from . import attention, tuned
-    lookup = lookup or tuned.lookup
+    lookup = lookup or (lambda name, shape: tuned.lookup(name, shape, space=space_of(name)))
     search = search or (lambda kind, shape: attention.autotune(kind, shape, verbose=True)[:2])
-    record = record or (lambda name, shape, config: tuned.record(name, shape, config, store=store))
+    record = record or (lambda name, shape, config: tuned.record(name, shape, config, store=store,
+                                                                 space=space_of(name)))
     done = {}
     for name, kind, shape in jobs(micro_batch, seq_len, cfg):
         if not force and lookup(name, shape) is not None:
@@ -107,8 +114,8 @@ def main(argv=None):
     print(f"tuning on {tuned.device_key()}")
     print(f"store: {store}\n")
 
-    def lookup(name, shape):   # only what the target store already holds counts as known
-        return tuned._read(store).get(tuned.device_key(), {}).get(tuned._shape_key(name, shape))
+    def lookup(name, shape):   # only what the target store holds, chosen from this build's tilings, counts as known
+        return tuned.known(store, name, shape, space_of(name))
 
     ok = True
     for name, micro, seq in shapes:

@@ -17,7 +17,10 @@ Two files are consulted, this machine's own store first:
   search.
 
 A device missing from both simply misses: its kernels search (``AUTOTUNE``)
-or use the defaults, never tiles measured on other hardware.
+or use the defaults, never tiles measured on other hardware.  A record of the
+store also names the set of tilings it was chosen from: where a search can run,
+one that an earlier build made over another set misses, so that tilings added
+since are timed; elsewhere it still serves.
 
     python -m mimansm1_v1_amd.tune      # fill the store for the run's shapes
     python -m mimansm1_v1_amd.tuned     # show what is remembered
@@ -32,6 +35,7 @@ from pathlib import Path
 TABLE = Path(__file__).with_name("tuned_tiles.json")
 STORE = Path(os.environ.get("MM1_TUNED_STORE",
                             Path.home() / ".cache" / "mimansm1_v1_amd" / "tuned_tiles.json"))
+SPACE = "tile_space"     # field of a record: the tilings it was chosen from
 _lock = threading.Lock()
 
 
@@ -61,21 +65,35 @@ def _read(path: Path) -> dict:
         return {}
 
 
-def lookup(kernel: str, shape, device: str | None = None):
-    """The remembered config for this kernel and shape, or None."""
+def _entry(path, kernel, shape, device, space):
+    hit = _read(path).get(device, {}).get(_shape_key(kernel, shape))
+    if not hit or (space is not None and hit.get(SPACE) != space):
+        return None
+    return {name: value for name, value in hit.items() if name != SPACE}
+
+
+def lookup(kernel: str, shape, device: str | None = None, space: str | None = None):
+    """The remembered config for this kernel and shape, or None.  With `space`,
+    a record of the store counts only if it was chosen from that set of tilings
+    (the shipped table belongs to the build and always counts)."""
     device = device or device_key()
-    key = _shape_key(kernel, shape)
-    for path in (STORE, TABLE):
-        hit = _read(path).get(device, {}).get(key)
-        if hit:
-            return dict(hit)
-    return None
+    return _entry(STORE, kernel, shape, device, space) or _entry(TABLE, kernel, shape, device, None)
 
 
-def record(kernel: str, shape, config: dict, device: str | None = None, store=None) -> None:
-    """Remember a tuned config (written at once; empty configs are ignored)."""
+def known(store, kernel: str, shape, space: str):
+    """The config that `store` holds for this kernel and shape on this device,
+    chosen from the tilings `space`, or None."""
+    return _entry(store, kernel, shape, device_key(), space)
+
+
+def record(kernel: str, shape, config: dict, device: str | None = None, store=None,
+           space: str | None = None) -> None:
+    """Remember a tuned config, chosen from the tilings `space` (written at
+    once; empty configs are ignored)."""
     if not config:
         return
+    if space is not None:
+        config = {**config, SPACE: space}
     path = Path(store or STORE)
     device = device or device_key()
     with _lock:

@@ -178,6 +178,43 @@ def test_get_kernel_uses_record_and_ignores_stale_one(tmp_path, monkeypatch):
     assert A.get_kernel("bwd", *shape).config == A.BWD_TILES     # no GPU: defaults
 
 
+@pytest.mark.parametrize("kind", ["fwd", "bwd"])
+def test_a_record_from_another_set_of_tilings_is_searched_again(tmp_path, monkeypatch, kind):
+    """A record that an earlier build chose from fewer tilings, or without saying
+    from which, misses where a search can run, and the search's record replaces
+    it and serves from then on; without a search it still serves."""
+    monkeypatch.setattr(tuned, "STORE", tmp_path / "store.json")
+    monkeypatch.setattr(tuned, "TABLE", tmp_path / "none.json")
+    monkeypatch.setattr(tuned, "device_key", lambda: "gfx950-256cu")
+    shape, name = (3, 10, 96, 128, True, 5), f"attention_{kind}"
+    configs = A.fwd_configs() if kind == "fwd" else A.bwd_configs()
+    old, new, searches = configs[1], configs[-1], []
+    with monkeypatch.context() as m:
+        m.setattr(A, "tile_space", lambda part, full=A.tile_space: full(part)[:-1])
+        smaller = A.tile_space_id(kind)
+    assert smaller != A.tile_space_id(kind) == A.tile_space_id(kind)
+
+    def handle():
+        monkeypatch.setattr(A, "_kernels", {})
+        return A.get_kernel(kind, *shape)
+
+    for space in (smaller, None):
+        tuned.record(name, shape, old, space=space)
+        assert handle().config == old                       # AUTOTUNE off
+        with monkeypatch.context() as m:
+            m.setattr(A, "AUTOTUNE", True)
+            m.setattr(torch.cuda, "is_available", lambda: True)
+            m.setattr(A, "autotune", lambda k, s: (searches.append(s), (new, 1.0, []))[1])
+            assert handle().config == new == handle().config
+        assert searches == [shape] and tuned.lookup(name, shape) == new
+        searches.clear()
+    # the tune command counts a record as known by the same rule
+    from mimansm1_v1_amd import tune as T
+    assert tuned.known(tuned.STORE, name, shape, T.space_of(name)) == new
+    tuned.record(name, shape, old, space=smaller)
+    assert tuned.known(tuned.STORE, name, shape, T.space_of(name)) is None
+
+
 def test_shipped_tile_table_names_compiled_tilings():
     """The measured gfx950 table covers both run shapes, fwd and bwd, and every
     entry is a tiling this build has."""
