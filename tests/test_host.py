@@ -402,3 +402,33 @@ def test_tied_head_wide_embeddings_go_through_the_transposed_copy(monkeypatch, d
     assert tuple(weight.shape) == ((384, d) if kind == "rows" else (d, 384))
     if kind == "columns":
         assert weight.dtype == torch.bfloat16 and weight.is_contiguous()
+
+
+ROW, COL = 0, 1
+
+
+@pytest.mark.parametrize("m,n,k,x,w,joined,faster", [
+    # x k-contiguous, a long reduction: split over idle CUs, or the library's tiles fill the round
+    (1024, 1280, 49152, ROW, ROW, False, True), (1024, 1280, 49152, ROW, COL, False, True),
+    (2048, 512, 49152, ROW, ROW, False, True), (8192, 1280, 49152, ROW, ROW, False, False),
+    (9741, 1280, 32000, ROW, COL, False, False), (12288, 512, 49152, ROW, ROW, False, False),
+    (16384, 1280, 49152, ROW, ROW, False, True), (430, 1280, 49152, ROW, ROW, False, False),
+    # rounds of 320-column tiles
+    (16384, 1280, 1280, ROW, ROW, False, True), (65536, 1280, 1280, ROW, ROW, False, False),
+    (18000, 1280, 1280, ROW, ROW, False, False), (32768, 1280, 1280, ROW, ROW, False, True),
+    (16384, 5120, 2048, ROW, ROW, False, False), (16384, 4480, 2048, ROW, ROW, False, True),
+    (16384, 1280, 3328, ROW, COL, False, True), (5662, 1280, 3328, ROW, COL, False, False),
+    (3562, 2048, 4352, ROW, COL, False, False), (9741, 1280, 8192, ROW, COL, False, False),
+    (13312, 1280, 8192, ROW, ROW, False, False), (13777, 1280, 8192, ROW, COL, False, True),
+    (16384, 1280, 6656, ROW, ROW, True, True), (8192, 1280, 6656, ROW, ROW, True, False),
+    # weight gradients
+    (1280, 6656, 16384, COL, COL, False, True), (8192, 1280, 8192, COL, COL, False, False),
+    (1280, 8192, 8192, COL, COL, False, False), (1280, 8192, 2455, COL, COL, False, True),
+    (8192, 1280, 16384, COL, COL, False, True), (49152, 1280, 8192, COL, COL, False, True),
+    # too few products
+    (1792, 1280, 4096, COL, COL, False, False), (4096, 1280, 1280, ROW, COL, False, False)])
+def test_products_run_where_they_were_measured_faster(m, n, k, x, w, joined, faster):
+    """The size rule of the GEMM core against hipBLASLt, on both sides of each of
+    its lines, at products whose two times were measured."""
+    from mimansm1_v1_amd import gemm
+    assert gemm.pays(m, n, k, x, w, joined) is faster
