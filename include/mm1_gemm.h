@@ -24,9 +24,9 @@ extern "C" {
 #define MM1_GEMM_ROW 0
 #define MM1_GEMM_COL 1
 
-/* Bytes of scratch mm1_gemm needs for this shape, with (joined) or without a
- * w1 (0 for many): fp32 partial
- * sums where K is split over several workgroups. */
+/* Bytes of scratch mm1_gemm needs for this shape in any layouts, with (joined)
+ * or without a w1 (0 for many): fp32 partial sums where K is split over several
+ * workgroups. */
 size_t mm1_gemm_workspace_size(int M, int N, int K, int joined);
 
 /* Modelled time of mm1_gemm at this shape on the current device, in us

@@ -692,7 +692,10 @@ static bool gemm_sizes_ok(int M, int N, int K) {
 }
 
 size_t mm1_gemm_workspace_size(int M, int N, int K, int joined) {
-  return gemm_sizes_ok(M, N, K) ? mm1::gemm_workspace_bytes(M, N, K, joined != 0) : 0;
+  if (!gemm_sizes_ok(M, N, K)) return 0;
+  const size_t rows = mm1::gemm_workspace_bytes(M, N, K, false, joined != 0);     // enough for any layouts
+  const size_t k_major = mm1::gemm_workspace_bytes(M, N, K, true, joined != 0);
+  return rows > k_major ? rows : k_major;
 }
 
 double mm1_gemm_estimate_us(int M, int N, int K) { return gemm_sizes_ok(M, N, K) ? mm1::gemm_estimate_us(M, N, K) : -1.; }
@@ -714,7 +717,7 @@ int mm1_gemm(const void* x, int x_layout, long ldx, const void* w, int w_layout,
   if (!aligned16(x) || !aligned16(w) || (w1 && !aligned16(w1)) || !aligned16(out) || (out1 && !aligned16(out1)) ||
       (workspace && !aligned16(workspace)))
     return MM1_E_ALIGN;
-  const size_t need = mm1::gemm_workspace_bytes(M, N, K, w1 != nullptr);
+  const size_t need = mm1::gemm_workspace_bytes(M, N, K, xc, w1 != nullptr);
   if (need > 0 && (!workspace || workspace_bytes < need)) return MM1_E_WORKSPACE;
   mm1::GemmArgs a{x, ldx, x_layout, w, ldw, w_layout, w1, k_cut, out, out1, n_cut, ldo, out_f32 != 0, workspace, M, N, K};
   return from_hip(mm1::launch_gemm(a, static_cast<hipStream_t>(stream)));

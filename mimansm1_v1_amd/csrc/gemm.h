@@ -24,7 +24,7 @@ struct GemmArgs {
 };
 
 bool gemm_operand_fits(int layout, long ld, int n, int K);
-size_t gemm_workspace_bytes(int M, int N, int K, bool joined);
+size_t gemm_workspace_bytes(int M, int N, int K, bool k_major, bool joined);
 double gemm_estimate_us(int M, int N, int K);
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t stream);
 

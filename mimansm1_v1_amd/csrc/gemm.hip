@@ -223,7 +223,8 @@ namespace {
 // Cost of a plan in windows of a 256-column tile (~1.4 us each).
 constexpr double SPLIT_COST = 28;   // writing the partial sums and adding them: ~40 us, measured at 65 to 320 tiles
 constexpr double FILL_COST = 7;     // launch, first window and epilogue, 10 us
-constexpr double HALF_COST = 0.85;  // a half tile (WholeTiles): its copies are a whole tile's
+constexpr double HALF_COST = 0.85;  // a half tile (WholeTiles), whose copies are a whole tile's, or a whole tile of
+                                    // a k-contiguous x with half of the CUs idle (plan_of)
 
 // Small tiles, in us: the launch and the ring's first fill, each round of
 // workgroups, each of its windows, and the sum of the splits.
@@ -237,7 +238,12 @@ struct Plan {
   size_t part_bytes;
 };
 
-Plan plan_of(int bn, int M, int N, int K, int n_g) {
+// A last round of tiles for at most half of the CUs: half tiles after full
+// rounds; alone, whole tiles, which run faster than in a full round with x
+// k-contiguous (5662 x 1280 x 3328, 115 tiles: 63 us whole, 79 split along k; 3584 x
+// 2048 x 4096, 112 tiles: 86, 96) but not with both operands k-major (4096 x 2048
+// x 4937, 128 tiles: 122, 93; x 4096 100, 85).
+Plan plan_of(int bn, int M, int N, int K, bool k_major, int n_g) {
   Plan p{};
   p.wide320 = bn == 320;
   p.n_mblk = (M + gemm::BM - 1) / gemm::BM;
@@ -245,7 +251,7 @@ Plan plan_of(int bn, int M, int N, int K, int n_g) {
   const long total = (long)p.n_mblk * p.n_nblk;
   const int left = (int)(total % n_g);
   const double tile = (double)gemm::windows_of(K) * bn / 256, full = (double)(total / n_g);
-  const double last = left == 0 ? 0 : 2 * left <= n_g ? HALF_COST : 1;
+  const double last = left == 0 ? 0 : 2 * left <= n_g && (total > n_g || !k_major) ? HALF_COST : 1;
   p.cost = FILL_COST + (full + last) * tile;
   p.grid = gemm::persistent_grid(n_g, (int)total);
   const double split = FILL_COST + (full + (double)left / n_g) * tile + SPLIT_COST;
@@ -284,9 +290,11 @@ Plan small_plan(int M, int N, int K, int n_g) {
 }
 
 // The tile size, and the split of the leftover tiles or of k, by modelled cost.
-Plan make_plan(int M, int N, int K, int cus, bool joined) {
+// k_major: both operands are.
+Plan make_plan(int M, int N, int K, bool k_major, int cus, bool joined) {
   const int n_g = ((cus > 0 ? cus : 256) + 7) & ~7;
-  const Plan a = plan_of(256, M, N, K, n_g), b = plan_of(320, M, N, K, n_g), c = small_plan(M, N, K, n_g);
+  const Plan a = plan_of(256, M, N, K, k_major, n_g), b = plan_of(320, M, N, K, k_major, n_g);
+  const Plan c = small_plan(M, N, K, n_g);
   const Plan& large = b.cost < a.cost ? b : a;
   return c.cost < large.cost && !joined ? c : large;      // the small tiles take one W only
 }
@@ -371,23 +379,23 @@ bool gemm_operand_fits(int layout, long ld, int n, int K) {
   return gemm::offsets_fit(static_cast<gemm::Layout>(layout), ld, n, K);
 }
 
-size_t gemm_workspace_bytes(int M, int N, int K, bool joined) {
+size_t gemm_workspace_bytes(int M, int N, int K, bool k_major, bool joined) {
   int cus = 0;
   if (cu_count(cus) != hipSuccess) cus = 256;
-  return make_plan(M, N, K, cus, joined).part_bytes;
+  return make_plan(M, N, K, k_major, cus, joined).part_bytes;
 }
 
 double gemm_estimate_us(int M, int N, int K) {
   int cus = 0;
   if (cu_count(cus) != hipSuccess) cus = 256;
-  return make_plan(M, N, K, cus, false).cost * WINDOW_US;
+  return make_plan(M, N, K, false, cus, false).cost * WINDOW_US;
 }
 
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t stream) {
   int cus = 0;
   hipError_t e = cu_count(cus);
   if (e != hipSuccess) return e;
-  const Plan plan = make_plan(a.M, a.N, a.K, cus, a.w1 != nullptr);
+  const Plan plan = make_plan(a.M, a.N, a.K, a.x_layout == gemm::COL, cus, a.w1 != nullptr);
   const gemm::Problem p{{static_cast<const __bf16*>(a.x), a.ldx, a.M}, {static_cast<const __bf16*>(a.w), a.ldw, a.N},
                         static_cast<const __bf16*>(a.w1), a.k_cut, a.K, plan.n_mblk, plan.n_nblk};
   const Output o{a.out, a.out1, a.ldo, a.M, a.N, a.out1 ? a.n_cut : a.N};

@@ -400,6 +400,18 @@ def test_lm_head_rows_entries_bound_the_width(lib, d, fits):
     assert L.rows_apply(d) is fits
 
 
+def test_gemm_splits_a_lone_round_of_k_major_tiles(lib):
+    """Without a device the plans are those of 256 CUs.  A lone round of at most
+    half of them is split along k where both operands may be k-major: the
+    scratch holds a partial tile of every workgroup and one more per tile."""
+    tile = 256 * 256 * 4
+    assert lib.mm1_gemm_workspace_size(4096, 2048, 4937, 0) == (256 + 128) * tile
+    assert lib.mm1_gemm_workspace_size(3584, 2048, 4096, 0) == (256 + 112) * tile
+    assert lib.mm1_gemm_workspace_size(3328, 1280, 8192, 0) == (256 + 65) * tile       # split in any layout
+    assert lib.mm1_gemm_workspace_size(4096, 2048, 2048, 0) == 0                       # shorter: whole tiles
+    assert lib.mm1_gemm_workspace_size(4096, 4096, 4096, 0) == 0                       # every CU has a tile
+
+
 # ---------------------------------------------------------------------------
 # Workgroup dispatch order of the causal grids (host-side model, no device).
 

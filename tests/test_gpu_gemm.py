@@ -49,6 +49,15 @@ def test_products_vs_fp64(hip_device, M, N, K, layout):
         assert torch.equal(out, gemm.product(x, w, out_dtype=dtype))
 
 
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+def test_plan_that_depends_on_the_layout(hip_device, layout):
+    """112 tiles: whole ones with x k-contiguous, split along k with both k-major."""
+    gen = torch.Generator(device=hip_device).manual_seed(5)
+    x, w = operand(3584, 4096, layout == "tn", gen, hip_device), operand(2048, 4096, layout != "nt", gen, hip_device)
+    for dtype in (torch.bfloat16, torch.float32):
+        check(gemm.product(x, w, out_dtype=dtype), x, w)
+
+
 @pytest.mark.parametrize("M", [1, 77, 255, 257, 333])
 def test_ragged_rows_and_padded_strides(hip_device, M):
     gen = torch.Generator(device=hip_device).manual_seed(M)
