@@ -58,6 +58,21 @@ def test_plan_that_depends_on_the_layout(hip_device, layout):
         check(gemm.product(x, w, out_dtype=dtype), x, w)
 
 
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("M,N,K,dtype", [(62608, 1608, 128, torch.bfloat16), (78648, 1280, 128, torch.bfloat16),
+                                         (33352, 1608, 128, torch.float32), (31304, 1608, 128, torch.float32),
+                                         (12088, 8328, 4096, torch.bfloat16), (32952, 3200, 4096, torch.bfloat16),
+                                         (39328, 1280, 4096, torch.float32), (15736, 3200, 4096, torch.float32)])
+def test_outputs_past_the_caches(hip_device, M, N, K, dtype, layout):
+    """Above 192 MiB the output leaves with non-temporal stores: tiles of 256 and
+    of 320 columns (in pairs), whole and, from the fifth on, split along k."""
+    assert M * N * dtype.itemsize > 192 << 20
+    assert (_lib.load().mm1_gemm_workspace_size(M, N, K, 0) > 0) == (K == 4096)
+    gen = torch.Generator(device=hip_device).manual_seed(M + N)
+    x, w = operand(M, K, layout == "tn", gen, hip_device), operand(N, K, layout != "nt", gen, hip_device)
+    check(gemm.product(x, w, out_dtype=dtype), x, w)
+
+
 @pytest.mark.parametrize("M", [1, 77, 255, 257, 333])
 def test_ragged_rows_and_padded_strides(hip_device, M):
     gen = torch.Generator(device=hip_device).manual_seed(M)

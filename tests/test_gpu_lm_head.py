@@ -178,3 +178,21 @@ def test_tied_head_holds_its_own_bf16_matrix(hip_device, chunk):
         loss.backward()
         results.append((loss.detach(), hid.grad, emb.weight.grad))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("rows", [False, True])
+def test_dlogits_past_the_caches(hip_device, rows):
+    """Above 192 MiB the d_logits leave with non-temporal stores: bitwise those of
+    two chunks below it, with the weight by columns and by rows, ragged tokens."""
+    from mimansm1_v1_amd import lm_head as L
+    T, d, V = 2100, 128, 49152
+    assert T * V * 2 > 192 << 20 > T * V
+    h, w, t = (x.to(hip_device) for x in LMO.make_inputs(T, d, V, seed=9, h_std=1.0, w_std=0.05, n_ignore=7))
+    kernel = L.get_kernel((T, d, V))
+    w = w.t().contiguous() if rows else w
+    lse = (kernel.forward_rows if rows else kernel.forward)(h, w, t)[0]
+    dlogits = kernel.dlogits_rows if rows else kernel.dlogits
+    scale = torch.full((1,), 1.0 / T, device=hip_device)
+    whole = dlogits(h, w, t, lse, scale, 0, V)
+    for v0 in (0, V // 2):
+        assert torch.equal(whole[:, v0:v0 + V // 2], dlogits(h, w, t, lse, scale, v0, V // 2))

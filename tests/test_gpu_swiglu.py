@@ -176,3 +176,47 @@ def test_few_tokens_and_the_act_alone(hip_device, T, d, Fh):
     with torch.no_grad():
         assert torch.equal(out, S.fused_swiglu(x, wg, wu, w_down))
     assert torch.equal(out, kept.detach()) and kept.requires_grad and not out.requires_grad
+
+
+@pytest.mark.parametrize("kind,outputs,T", [("train", 3, 10244), ("split", 2, 15364), ("gate_up", 1, 30724), ("act", 1, 30724)])
+def test_outputs_past_the_caches(hip_device, kind, outputs, T):
+    """Outputs above 192 MiB leave with non-temporal stores: bitwise those of two
+    halves of the tokens, which are below it."""
+    from mimansm1_v1_amd import swiglu as S
+    d, Fh, cut = 128, 3328, T // 512 * 256
+    assert outputs * T * Fh * 2 > 192 << 20 > outputs * (T - cut) * Fh * 2
+    gen = torch.Generator(device=hip_device).manual_seed(T)
+    x = torch.randn(T, d, device=hip_device, generator=gen).to(torch.bfloat16)
+    wg, wu = ((torch.randn(d, Fh, device=hip_device, generator=gen) * 0.05).to(torch.bfloat16) for _ in range(2))
+
+    def run(rows):
+        if kind == "act":
+            return (S.get_kernel("train", rows.shape[0], d, Fh).act_only(rows, wg, wu),)
+        out = S.get_kernel(kind, rows.shape[0], d, Fh)(rows, wg, wu)
+        return out if isinstance(out, tuple) else (out,)
+
+    whole, lo, hi = run(x), run(x[:cut]), run(x[cut:])
+    assert len(whole) == outputs
+    for a, b, c in zip(whole, lo, hi):
+        assert torch.equal(a, torch.cat((b, c)))
+
+
+def test_backward_on_the_core(hip_device, monkeypatch):
+    """At 14,848 tokens every product of the backward but d_act, the joined d_x
+    among them, runs on the GEMM core: the gradients are those of torch's products
+    up to the bf16 roundings on the way (d_x: one against two)."""
+    from mimansm1_v1_amd import gemm, swiglu as S
+    T, d, Fh = 14848, 1280, 1280
+    gen = torch.Generator(device=hip_device).manual_seed(1)
+    rand = lambda *shape, std=1.0: (torch.randn(*shape, device=hip_device, generator=gen) * std).to(torch.bfloat16)
+    leaves = [t.requires_grad_(True) for t in (rand(T, d), rand(d, Fh, std=0.03), rand(d, Fh, std=0.03), rand(Fh, d, std=0.03))]
+    dy, taken = rand(T, d), []
+    for name in ("applies", "applies_joined"):
+        real = getattr(gemm, name)
+        monkeypatch.setattr(gemm, name, lambda *a, real=real, name=name: (taken.append((name, real(*a))), taken[-1][1])[1])
+    got = torch.autograd.grad(S.fused_swiglu(*leaves), leaves, dy)
+    assert taken.count(("applies_joined", True)) == 1 and taken.count(("applies", True)) >= 3
+    for name in ("applies", "applies_joined"):
+        monkeypatch.setattr(gemm, name, lambda *a: False)
+    for a, b in zip(got, torch.autograd.grad(S.fused_swiglu(*leaves), leaves, dy)):
+        assert (a.double() - b.double()).norm() <= 2.0 ** -7 * b.double().norm()
