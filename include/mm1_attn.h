@@ -243,7 +243,8 @@ int mm1_attn_bwd_f32_tiles(const void* o, const void* dO, const float* lse2,
  *  - mm1_attn_tile_count(kind): number of tilings of MM1_TILES_FWD,
  *    MM1_TILES_DKDV or MM1_TILES_DQ (0 for another kind);
  *  - mm1_attn_tile_desc(kind, i): static "key=value ..." description of
- *    tiling i (block_M, block_N, waves, stages, schedule), NULL if out of range.
+ *    tiling i (block_M, block_N, waves, stages, schedule), NULL if out of range;
+ *    block_N is the rows of one streamed LDS tile (a "keysplit" step takes two).
  * Index 0 is each kind's default, which the calls without a tiling argument
  * use. */
 int mm1_attn_tile_count(int kind);

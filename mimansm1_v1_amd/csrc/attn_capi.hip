@@ -73,8 +73,9 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 // Tilings compiled into the library (the `variant` argument of launch_fwd,
 // launch_bwd_dkdv and launch_bwd_dq).  block_M / block_N name the stationary
-// and the streamed block: query rows x key rows for the forward and dQ, key
-// rows x query rows for dK/dV.
+// and the streamed block (one LDS tile; a keysplit step takes two, SPLIT_KEYS
+// keys): query rows x key rows for the forward and dQ, key rows x query rows for
+// dK/dV.
 const char* const kFwdTiles[] = {
     "block_M=256 block_N=64 waves=8 stages=2 schedule=pingpong",
     "block_M=128 block_N=64 waves=4 stages=2 schedule=ring",

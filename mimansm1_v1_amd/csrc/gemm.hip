@@ -8,10 +8,10 @@
 // with either operand ROW (k contiguous) or COL (k-major).  W may be two
 // matrices joined along k, and the output two matrices joined along n.
 //
-// Tiles are 256 x 256, one workgroup per CU.  Where the tile count leaves a
+// Tiles are 256 x 256 or 256 x 320, one workgroup per CU.  Where the tile count leaves a
 // last round mostly empty and the reduction is long, the leftover tiles are
 // split along k over all workgroups (SplitTiles): each workgroup writes its
-// fp32 partial tiles (at most two, 256 KiB each) and split_sum_kernel adds
+// fp32 partial tiles (at most two, 256 or 320 KiB each) and split_sum_kernel adds
 // them in a fixed order and rounds once, so results are deterministic.
 #include <hip/hip_runtime.h>
 
@@ -175,8 +175,8 @@ __global__ __launch_bounds__(64 * S::TI) void split_sum_kernel(const float* __re
 // workgroups on consecutive items; with several splits of k each writes its
 // fp32 partial tile ([wave][q][lane] x 4 floats) to slot tile * splits + split
 // and small_sum_kernel adds them in split order.  Bound by the latency of one
-// tile's k walk (0.35 us a window): 77 x 3328 x 1280 12.1 us a call, 300 x 1280 x
-// 1280 11.3, 77 x 1280 x 6656 (15 splits) 15.5, where torch's GEMM takes 21 us
+// tile's k walk (0.35 us a window): 77 x 3328 x 1280 10.6 us a call, 300 x 1280 x
+// 1280 10.5, 77 x 1280 x 6656 (6 splits) 14.9, where torch's GEMM takes 20.6 to 23
 // (its host work).
 template <gemm::Layout LX, gemm::Layout LW, bool F32>
 __global__ __launch_bounds__(256) void gemm_small_kernel(const gemm::Problem p, const Output o, float* part,

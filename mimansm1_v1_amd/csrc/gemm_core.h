@@ -1,23 +1,24 @@
 // Persistent bf16 GEMM core for gfx950 shared by the SwiGLU and LM-head
 // kernels and the plain products around them: D[m][n] = sum_k X(m, k) W(n, k)
-// in tiles of 256 rows x 256 columns, fp32 accumulation, with the epilogue
-// supplied by the caller.
+// in tiles of 256 rows x BN (256 or 320) columns, fp32 accumulation, with the
+// epilogue supplied by the caller.
 //
 // Either operand is ROW (k contiguous: X [M, K], W [N, K]) or COL (k-major:
 // X [K, M], W [K, N]); PAIRED takes W's columns from two COL matrices (128
 // columns of each per tile: the SwiGLU gate and up weights).
 //
 // A workgroup (8 waves, two per SIMD, one workgroup per CU) owns a tile and
-// walks k in windows of 64 staged in a two-slot LDS ring (64 KiB per slot) by
-// the LDS DMA.  Wave (wm, wn), wm = w % WM, wn = w / WM, accumulates TI row
+// walks k in windows of 64 staged in a two-slot LDS ring (64 or 72 KiB per slot)
+// by the LDS DMA.  Wave (wm, wn), wm = w % WM, wn = w / WM, accumulates TI row
 // blocks of 32 from block TI wm on against the TJ column blocks from TJ wn on
 // or (PAIRED) block wn of the first and of the second matrix.  acc[b][i] is
 // the 32 x 32 product of column block b and row block i (lane: row 32i +
 // (lane & 31); register 4q + e: column 8q + 4(lane/32) + e of the block).
 //
 // What bounds it, and the layout that follows from it.  The products alone
-// run at 1.79 PFLOP/s here (the clock falls to ~1.75 GHz under them); the
-// L1 / L2 path that feeds the ring is the next limit, so:
+// run at 1.79 PFLOP/s here (the clock falls to ~1.75 GHz under them); timing
+// copies made the path that feeds the ring the next limit (8192^3 now 1.24-1.39
+// PFLOP/s by layout; hipBLASLt 1.61, 1.42 and 1.23), so:
 //   * every copy moves whole 128-byte lines (64 k of one row, or 64 columns
 //     of one k): with 64-byte pieces (32 k per window) the copies alone took
 //     1500 clocks per 32 k and the 8192^3 products ran at 1.22-1.25 PFLOP/s;
@@ -269,7 +270,7 @@ struct SplitTiles {
 // The persistent loop of one workgroup (512 threads, all of which must call
 // it), over the items of Tiles; pro(mb, nb) runs in each item's first window
 // (its loads land during the products), epi(mb, nb, acc, part) at its end
-// with acc[2][4] as described above.
+// with acc[TJ][TI] as described above.
 template <Layout LX, Layout LW, bool PAIRED, class S, class Tiles, class Pro, class Epi>
 __device__ __forceinline__ void run(const Problem& p, char* smem, Pro&& pro, Epi&& epi) {
   static_assert(!PAIRED || (LW == COL && std::is_same<S, Wide256>::value), "paired weights are k-major");
