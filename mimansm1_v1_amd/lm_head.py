@@ -246,19 +246,27 @@ def rows_apply(d_model) -> bool:
     return 257 * d_model < 1 << 30
 
 
+def _own_copy(embedding):
+    """A bf16 copy in every dtype: the backward's matrix stays the forward's when
+    the embedding changes in between, and the kernels take any embedding's alignment."""
+    return embedding.to(DTYPE, copy=True, memory_format=torch.contiguous_format)
+
+
 class TiedCrossEntropy(torch.autograd.Function):
     """FusedCrossEntropy for a head tied to its embedding: `embedding` is the
     [V, d] matrix as it lies in memory, which the kernels read by rows, so no
     transposed copy is made (at V 49152, d 1280 the transpose alone took 255
     us), and its gradient leaves the product in the embedding's own layout and
     dtype (fp32 sums, rounded once or not at all).  `weight` is the embedding's
-    bf16 copy, an input of its own so that a recorded backward's d_hidden
-    stays connected to the embedding; its gradient goes to `embedding`."""
+    bf16 copy (_own_copy), an input of its own so that a recorded backward's
+    d_hidden stays connected to the embedding; its gradient goes to
+    `embedding`.  Without it the copy is made here, unconnected."""
 
     @staticmethod
-    def forward(ctx, hidden, embedding, weight, targets, chunk):
+    def forward(ctx, hidden, embedding, targets, chunk, weight=None):
         tokens, d_model = hidden.shape
         vocab = embedding.shape[0]
+        weight = _own_copy(embedding) if weight is None else weight
         _check_bf16_hip(hidden, weight)
         kernel = get_kernel((tokens, d_model, vocab))
         targets = targets.contiguous()
@@ -292,10 +300,7 @@ class TiedCrossEntropy(torch.autograd.Function):
 
 
 def tied_cross_entropy(hidden, embedding, targets, chunk=VOCAB_CHUNK):
-    # a copy in every dtype: the backward's matrix stays the forward's when the
-    # embedding changes in between, and the kernels take any embedding's alignment
-    weight = embedding.to(DTYPE, copy=True, memory_format=torch.contiguous_format)
-    return TiedCrossEntropy.apply(hidden, embedding, weight, targets, chunk)
+    return TiedCrossEntropy.apply(hidden, embedding, targets, chunk, _own_copy(embedding))
 
 
 def fused_cross_entropy(hidden, weight, targets, chunk=VOCAB_CHUNK):

@@ -221,3 +221,7 @@ def test_recorded_backward_of_the_head(hip_device, T, monkeypatch):
     assert any(isinstance(g, tuple) for g in want)
     _same_terms(got, want)
     _same_terms(tied, copied)
+    # without its copy the Function makes one: the same first gradients
+    own = torch.autograd.grad(L.TiedCrossEntropy.apply(h, emb, t, 49152), [h, emb])
+    for a, b in zip(own, torch.autograd.grad(L.tied_cross_entropy(h, emb, t), [h, emb])):
+        assert torch.equal(a, b)
