@@ -352,11 +352,11 @@ class LMHead(nn.Module):
 
     def _loss_hip(self, rows, weight, targets):
         # bf16 kernels: the fp32 stream and matrix become contiguous bf16 here
-        # (LM:313-323); a tied matrix is read in the embedding's own layout, or,
-        # in widths beyond that kernel's offsets, from its transposed copy
+        # (LM:313-323); a tied matrix is read in the embedding's own layout (its
+        # transpose's transpose), or, in widths beyond that kernel's offsets, from
+        # its transposed copy
         if self.cfg.tied and rows_apply(self.cfg.d_model):
-            return tied_cross_entropy(rows.to(DTYPE).contiguous(), self.embedding[0].weight, targets,
-                                      self.cfg.chunk)
+            return tied_cross_entropy(rows.to(DTYPE).contiguous(), weight.t(), targets, self.cfg.chunk)
         return fused_cross_entropy(rows.to(DTYPE).contiguous(), weight.to(DTYPE).contiguous(), targets,
                                    self.cfg.chunk)
 

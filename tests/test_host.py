@@ -404,6 +404,26 @@ def test_tied_head_wide_embeddings_go_through_the_transposed_copy(monkeypatch, d
         assert weight.dtype == torch.bfloat16 and weight.is_contiguous()
 
 
+def test_tied_loss_takes_the_matrix_that_the_head_reports(monkeypatch):
+    """A head that derives its matrix from the embedding trains on that matrix:
+    the tied path gets matrix()'s transpose, connected to the embedding."""
+    from mimansm1_v1_amd import lm_head as L
+
+    class Scaled(L.LMHead):
+        def matrix(self):
+            return 2.0 * super().matrix()
+
+    monkeypatch.setattr(L, "tied_cross_entropy", lambda h, e, t, chunk: (h.float() @ e.t()).sum())
+    emb = torch.nn.Embedding(256, 128)
+    rows, targets = torch.ones(3, 128, dtype=torch.bfloat16), torch.zeros(3, dtype=torch.int64)
+    for head, factor in ((L.LMHead, 1.0), (Scaled, 2.0)):
+        emb.weight.grad = None
+        loss = head(L.HeadConfig(d_model=128, vocab=256, logit_scale=1.0), emb)(rows, targets)
+        torch.testing.assert_close(loss, factor * 3 * emb.weight.sum())
+        loss.backward()
+        torch.testing.assert_close(emb.weight.grad, torch.full_like(emb.weight, 3.0 * factor))
+
+
 ROW, COL = 0, 1
 
 
